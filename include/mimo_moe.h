@@ -25,14 +25,9 @@
  * written on the stream like every output (read it after the stream's work, no host sync inside the call);
  * NULL keeps it in the workspace.
  *
- * Streams: the prefill entry points (mimo_moe_prefill, mimo_moe_prefill_staged, mimo_moe_prefill_block,
- * mimo_moe_layer_prefill) run part of each grouped GEMM on a side stream forked from and joined back to
- * `stream` with events; every (device, stream) pair has its own side stream, kept for the life of the
- * process (the first 64 pairs; prefills on further streams run that part on `stream` itself, after the
- * rest, with the same results).  A call therefore orders work only on its own `stream`: prefills on different
- * streams never wait for each other, and a prefill captured into a HIP graph captures only its own stream's
- * work.  No entry point builds anything on the device at first use (the sigmoid table is constant data), so
- * the first call of a process may itself be captured.
+ * Streams: every entry point queues all of its work on `stream`: calls on different streams never wait for each
+ * other, and a call captured into a HIP graph captures only its own stream's work.  No entry point builds anything on
+ * the device at first use (the sigmoid table is constant data), so the first call of a process may itself be captured.
  */
 #ifndef MIMO_MOE_H
 #define MIMO_MOE_H
@@ -92,10 +87,9 @@ int mimo_random_bf16(uint64_t seed, float stddev, int64_t n, uint16_t* out, void
 int mimo_fill_random_mxfp4(uint64_t seed, float stddev, int64_t rows, int64_t cols, uint32_t* q, uint8_t* s,
                            void* stream);
 
-/* Activation split for the block-scaled MFMA paths: bf16 x [rows, cols] -> hi, lo E4M3 codes [rows, cols]
- * with E8M0 block scales hs, ls [rows, cols/32]; x == hi + lo for every element within 2^14 of its block
- * maximum.  Internal step of mimo_moe_experts / mimo_moe_prefill (the reference multiplies bf16
- * activations directly, kernels.py:59-68), exported for parity tests. */
+/* Two-plane E4M3 split of activations: bf16 x [rows, cols] -> hi, lo E4M3 codes [rows, cols] with E8M0 block scales
+ * hs, ls [rows, cols/32]; x == hi + lo for every element within 2^14 of its block maximum.  For callers that feed
+ * block-scaled FP8 MFMAs; no other entry point uses it. */
 int mimo_quantize_fp8_hilo(const uint16_t* x, int64_t rows, int64_t cols, uint8_t* hi, uint8_t* hs,
                            uint8_t* lo, uint8_t* ls, void* stream);
 
@@ -164,7 +158,7 @@ int mimo_moe_decode(const uint16_t* x, int M, const uint16_t* Wg, const float* b
 size_t mimo_moe_decode_workspace_size(int M, int E, int k, int H, int I);
 
 /* _moe_prefill (model.py:230-271) with every expert resident: slot_inds int32 [T, k] (slots), w fp32
- * [T, k]; sorted-by-slot grouped GEMMs on block-scaled MFMA, bf16 expert outputs, fixed-order weighted
+ * [T, k]; sorted-by-slot grouped GEMMs on bf16 MFMA, bf16 expert outputs, fixed-order weighted
  * combine.  y bf16 [T, H]; status_out (optional): MIMO_ERR_SLOT when a slot id is outside [0, n_slots). */
 int mimo_moe_prefill(const uint16_t* x, int T, const int32_t* slot_inds, const float* w, int k,
                      const mimo_bank* bank, uint16_t* y, int32_t* status_out, void* ws, size_t ws_bytes,

@@ -5,16 +5,13 @@
 // :198-199); _moe_small / _gather_m1 engine/mimo_stream/model.py:173-219.
 //
 // Each distinct expert's weights are streamed from HBM once and applied to every row routed to it.  The dot
-// products run on gfx950 block-scaled MFMA (v_mfma_scale_f32_16x16x128_f8f6f4): B = the expert's E2M1
-// weights with their E8M0 scales, exactly as stored; A = the activations split into hi + lo E4M3 halves
-// (each with its own E8M0 block scale) placed in MFMA rows 0-7 (hi) and 8-15 (lo), so one MFMA covers up to
-// eight token rows at bf16 precision and the two halves are summed in fp32 afterwards.
+// products run on v_mfma_f32_16x16x32_bf16: A = 16 weight rows, turned from E2M1 codes and E8M0 scales into bf16 in
+// registers (exactly), B = up to eight bf16 activation rows (columns 8-15 repeat them and are not used).
 //
-// MFMA operand layout (16x16x128, lane l: g = l / 16, i = l % 16), measured on MI355X:
-//   FP4 operand: lane holds K = 32g .. 32g+31 of row/column i (16 contiguous bytes).
-//   FP8 operand: bytes 0-15 hold K = 16g .. 16g+15, bytes 16-31 hold K = 64+16g .. 64+16g+15.
-//   scale of K-block b (32 wide) of row/column i comes from lane i + 16b (byte 0).
-//   D: lane l holds column l % 16, rows 4g .. 4g+3.
+// MFMA operand layout (16x16x32, lane l: g = l / 16, i = l % 16): both operands hold row/column i, 8 values of K
+// group g; D: lane l holds column l % 16, rows 4g .. 4g+3.  A K-step is 128 codes: a lane's 16 bytes of a weight row
+// are codes 32 g .. 32 g + 31 (one scale block), and MFMA m of the step takes codes 32 g + 8 m .. of every lane,
+// with the same columns of the activation rows.
 #include <atomic>
 #include <mutex>
 
@@ -27,7 +24,7 @@
 namespace mimo {
 
 struct ExpertsArgs {
-  const uint8_t *xq_hi, *xq_lo, *xq_hs, *xq_ls;   // [M, H], [M, H/32]
+  const uint16_t* x;                        // [M, H] bf16
   const uint32_t *gate_w, *up_w, *down_w;
   const uint8_t *gate_s, *up_s, *down_s;
   int H, I, R, Umax, k, M, S;
@@ -35,7 +32,6 @@ struct ExpertsArgs {
   const float* uw;
   const uint32_t* gidx;
   uint16_t* h;                              // [Umax, R, I] bf16
-  uint8_t *hq_hi, *hq_lo, *hq_hs, *hq_ls;   // [Umax, R, I], [Umax, R, I/32]
   float* part;                              // [Umax, R, H]
   int round_bf16, zero_pad;
   uint16_t* y;                              // [M, H]
@@ -52,100 +48,85 @@ struct ExpertsArgs {
   const uint16_t* resid;                    // [M, H] residual stream: y := bf16(resid + y) when given
 };
 
-// A operand (FP8 layout) for K-step k0 from a row of E4M3 codes; zero for padding rows.
-__device__ __forceinline__ v8i a_operand(const uint8_t* row, int k0, int g, bool valid) {
-  if (!valid) return v8i{0, 0, 0, 0, 0, 0, 0, 0};
-  uint4 a0 = *reinterpret_cast<const uint4*>(row + k0 + 16 * g);
-  uint4 a1 = *reinterpret_cast<const uint4*>(row + k0 + 64 + 16 * g);
-  return v8i{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
+// dword m of a lane's 16 bytes of codes: codes 32 g + 8 m .. of its row
+__device__ __forceinline__ uint32_t word_of(uint4 w, int m) { return m == 0 ? w.x : m == 1 ? w.y : m == 2 ? w.z : w.w; }
+// Whether one of 8 E8M0 bytes is 253 or 254: its weights can reach 2^128, which bf16 cannot hold.  A wave that meets
+// one multiplies with a quarter of every weight (then all fit) and takes its sums times 4.
+__device__ __forceinline__ bool has_huge_scale(uint2 v) {
+  auto word = [](uint32_t w) {     // bytes ^ 0xFE: 253 -> 3, 254 -> 0; and ^ 0xFD: 253 -> 0
+    const uint32_t a = w ^ 0xFEFEFEFEu, b = w ^ 0xFDFDFDFDu;
+    return (((a - 0x01010101u) & ~a) | ((b - 0x01010101u) & ~b)) & 0x80808080u;   // nonzero iff a zero byte
+  };
+  return (word(v.x) | word(v.y)) != 0u;
 }
-__device__ __forceinline__ v8i b_operand(uint4 b) { return v8i{(int)b.x, (int)b.y, (int)b.z, (int)b.w, 0, 0, 0, 0}; }
-
-#define MFMA_F8xF4(A, B, C, SA, SB) __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4((A), (B), (C), 0, 4, 0, (SA), 0, (SB))
+__device__ __forceinline__ bf16x8 lds_bf16x8(const uint8_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
 // ------------------------------------------------------------------ Kernel A: gate/up + SwiGLU
-// Block (512 threads): one distinct expert u (blockIdx.y) x 32 outputs n (blockIdx.x).  Wave w: 16-output
-// tile (w & 1) x K-range (w >> 1) of 4.  A wave's K-range is NS MFMA steps of K = 128 and its 2 x NS weight
-// loads (16 B of gate and of up per lane and step) are issued in one straight-line batch and stay in
-// registers, so a block keeps 8 x 16 KB of expert weights in flight.  Everything else the block reads is
-// requested before that batch: the expert's activation rows go straight to LDS (global_load_lds) and the
-// block's weight scales come in with one or two coalesced loads per thread; a load issued after the weight
-// batch would queue behind it.  Loads never depend on the lane: padding rows read row 0 and are zeroed by
-// selects.  K-range partials are summed in a fixed order through LDS; the epilogue applies the bf16 rounding
-// points of kernels.py:79-82 and writes the hi/lo split of h (and h itself when the caller asked for it).
+// Block (256 threads, four per CU): one distinct expert u (blockIdx.y) x 16 outputs n (blockIdx.x).  Wave w: K-range w
+// of 4.  A wave's K-range is NS K-steps of 128 codes and its 2 x NS weight loads (16 B of gate and of up per lane and
+// step) are issued in one straight-line batch and stay in registers, so a block keeps 4 x 16 KB of expert weights in
+// flight.  What bounds it is HBM: one block's conversions, MFMAs and epilogue run while the CU's three other blocks
+// load.  (Blocks of 512 threads and 32 outputs, two per CU, left more of that uncovered and spread a step's blocks less
+// evenly over the CUs: 4 rows of 23 experts 40.4 us against 36.1, 8 rows of 27 experts 59.5 against 54.7.)
+// Everything else the block reads is requested before that batch: the expert's activation rows go straight to LDS
+// (global_load_lds) and the block's weight scales come in with one or two coalesced loads per thread; a load issued
+// after the weight batch would queue behind it.  Loads never depend on the lane: columns without a row read row 0 of the staged ones
+// and their sums are dropped.  K-range partials are summed in a fixed order through LDS; the epilogue applies the bf16
+// rounding points of kernels.py:79-82 and writes h in bf16.
 __device__ __forceinline__ uint32_t byte_of(uint32_t w, int g) { return (w >> (8 * g)) & 0xFFu; }
 // K split of the gate/up reduction: 4 ranges when H % 512 == 0, else 2; MFMA steps (K = 128) per range.
 __host__ __device__ inline int gateup_ksplit(int H) { return H % 512 == 0 ? 4 : 2; }
 __host__ __device__ inline int gateup_steps(int H) { return H / gateup_ksplit(H) / 128; }
-__device__ __forceinline__ uint4 zero_if(uint4 v, bool keep) {
-  return keep ? v : make_uint4(0, 0, 0, 0);
-}
 __host__ __device__ constexpr int align_up(int x, int a) { return (x + a - 1) / a * a; }
 
 // Dynamic LDS of the gate/up kernel (bytes), for hidden size H and `rl` staged activation rows:
-//   scales  2 x 32 rows x RS       gate then up scales of the block's rows, RS = H/32 + 16 (conflict-free reads)
-//   a_hi    rl rows x RA           hi E4M3 codes of the staged rows, RA = H + 16 (rows 4 banks apart)
-//   a_lo    rl rows x RA           lo codes, starting 128 bytes off a_hi's bank phase
-//   a_sc    rl rows x 2 x H/32     [hi scales | lo scales] per row
-// The K-range partials and the h tile reuse the activation region once the MFMA loop is done.
+//   scales  2 x 16 rows x RS       gate then up scales of the block's rows, RS = H/32 + 16 (conflict-free reads)
+//   act     rl rows x RA           bf16 activation rows, RA = 2 H + 16 (rows 4 banks apart)
+// The K-range partials reuse the activation region once the MFMA loop is done.
 struct GateupLds {
-  int RS, RA, a_hi, a_lo, a_sc, red, hl, total;
+  int RS, RA, act, red, total;
 };
-constexpr int kRedBytes = 4 * 2 * 2 * 32 * 4 * 4;   // [K-range][ntile][gate/up][lane][q] floats
+constexpr int kRedBytes = 4 * 2 * 32 * 4 * 4;   // [K-range][gate/up][8 g + row][q] floats
 __host__ __device__ inline GateupLds gateup_lds(int H, int rl) {
   GateupLds L;
   L.RS = H / 32 + 16;
-  L.RA = H + 16;
-  L.a_hi = 2 * 32 * L.RS;
-  L.a_lo = align_up(L.a_hi + rl * L.RA, 256) + 128;
-  L.a_sc = align_up(L.a_lo + rl * L.RA, 16);
-  L.red = L.a_hi;
-  L.hl = L.red + kRedBytes;
-  const int a_end = L.a_sc + rl * 2 * (H / 32);
-  const int e_end = L.hl + 8 * 32 * 4;
+  L.RA = 2 * H + 16;
+  L.act = 2 * 16 * L.RS;
+  L.red = L.act;
+  const int a_end = L.act + rl * L.RA;
+  const int e_end = L.red + kRedBytes;
   L.total = a_end > e_end ? a_end : e_end;
   return L;
 }
 
-// Stage activation rows c0 .. c0 + n - 1 of the block's expert into LDS (rows 0 .. n - 1 there): per row, the
-// hi and lo codes in 1 KB pieces and the [hi | lo] scales in one piece, spread over the block's NW waves,
-// at most JMAX pieces per wave (n <= 8 rows of H <= 4096 need 9 with 8 waves).  Straight-line code: a loop here
-// would make the compiler drain every outstanding load before entering it.
+// Stage activation rows c0 .. c0 + n - 1 of the block's expert into LDS (rows 0 .. n - 1 there) in 1 KB pieces spread
+// over the block's four waves, at most JMAX pieces per wave (n <= 4 rows of H <= 4096 need 8).
+// Straight-line code: a loop here would make the compiler drain every outstanding load before entering it.
 // tok: lane c holds the token of row c (wave-uniform reads through readlane).
-template <int JMAX, int NW = 8>
+template <int JMAX>
 __device__ __forceinline__ void stage_act_rows(const ExpertsArgs& a, uint8_t* lds, const GateupLds& L, int c0, int n,
                                                int tok, int wave, int lane) {
-  const int nq = (a.H + 1023) >> 10;          // 1 KB pieces per half row
-  const int per_row = 2 * nq + 1;
-  const int hs = a.H / 32;
+  const int nq = (2 * a.H + 1023) >> 10;      // 1 KB pieces per row
 #pragma unroll
   for (int j = 0; j < JMAX; ++j) {
-    const int t = wave + NW * j;
-    if (t >= n * per_row) break;
-    const int c = t / per_row, p = t - c * per_row;
+    const int t = wave + 4 * j;
+    if (t >= n * nq) break;
+    const int c = t / nq, p = t - c * nq;
     int token = __builtin_amdgcn_readlane(tok, c0 + c);
     token = (token < 0 || token >= a.M) ? 0 : token;
-    if (p < 2 * nq) {
-      const int half = p >= nq, q = half ? p - nq : p;
-      const uint8_t* src = (half ? a.xq_lo : a.xq_hi) + (size_t)token * a.H + 1024 * q;
-      const uint8_t* dst = lds + (half ? L.a_lo : L.a_hi) + c * L.RA + 1024 * q;
-      if (1024 * q + 16 * lane < a.H) lds_copy16(src, 16 * lane, dst);
-    } else {                                      // [hi scales | lo scales] of the row, 4 bytes per lane
-      const uint8_t* dst = lds + L.a_sc + c * 2 * hs;
-      if (4 * lane < hs) lds_copy4(a.xq_hs + (size_t)token * hs, 4 * lane, dst);
-      else if (4 * lane < 2 * hs) lds_copy4(a.xq_ls + (size_t)token * hs - hs, 4 * lane, dst);
-    }
+    if (1024 * p + 16 * lane < 2 * a.H)
+      lds_copy16(reinterpret_cast<const uint8_t*>(a.x + (size_t)token * a.H) + 1024 * p, 16 * lane,
+                 lds + L.act + c * L.RA + 1024 * p);
   }
 }
 
-// Routes of one decode step for a block: wave r selects row r (top-k and renormalisation), wave 0 groups the
+// Routes of one decode step for a block: wave r selects rows r, r + 4 (top-k and renormalisation), wave 0 groups the
 // routes by slot (E <= 256).
 __device__ __forceinline__ void full_routing(const ExpertsArgs& a, int (*sel)[kSelLds], int32_t* s_inds, float* s_w,
                                              int* lurows, float* luw, int32_t* g_uids, int32_t* g_urows,
                                              int32_t* g_ucnt, float* g_uw, uint32_t* g_gidx, int32_t* g_nu, int wave) {
-  if (wave < a.M)
-    wave_select_row_t<4>(a.scores + wave * a.E, a.keys + wave * a.E, a.E, a.k, 1.0f, s_inds + wave * a.k,
-                         s_w + wave * a.k, sel[wave]);
+  for (int r = wave; r < a.M; r += 4)
+    wave_select_row_t<4>(a.scores + r * a.E, a.keys + r * a.E, a.E, a.k, 1.0f, s_inds + r * a.k, s_w + r * a.k, sel[r]);
   __syncthreads();
   if (wave == 0)
     wave_group_routes(s_inds, s_w, a.slot_of, a.M, a.k, a.R, a.S, a.Umax, g_uids, g_urows, g_ucnt, g_uw, g_gidx,
@@ -171,16 +152,8 @@ __device__ __forceinline__ void publish_routes(const ExpertsArgs& a, const int32
 }
 
 // FAST2 (routed only; the launcher checks its conditions): two rows with expert ids as slots.
-// HALF (the launcher uses it for one or two rows with expert ids as slots, where blocks take the fast selection):
-// blocks of 256 threads and 16 outputs (wave w: K-range w), four per CU, so that a step's U x I / 16 blocks spread
-// more evenly over the CUs than U x I / 32 larger ones; such a block writes h in bf16 and the down kernel splits
-// it (an E8M0 block of h spans 32 outputs, two of these blocks).
-template <int NS, bool ROUTED, bool FAST2, bool HALF = false>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) decode_gateup_kernel(ExpertsArgs a, int rl) {
-  static_assert(!HALF || ROUTED, "16-output blocks only for the routed kernel");
-  constexpr int NW = HALF ? 4 : 8;        // waves per block
-  constexpr int NT = HALF ? 1 : 2;        // 16-output tiles per block
-  constexpr int BO = 16 * NT;             // outputs per block
+template <int NS, bool ROUTED, bool FAST2>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) decode_gateup_kernel(ExpertsArgs a, int rl) {
   extern __shared__ __align__(16) uint8_t lds[];
   // routed grouping (ROUTED only): kept for the publication at the end of block (0, 0)
   __shared__ int sel[ROUTED ? 8 : 1][kSelLds];
@@ -191,6 +164,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) d
   __shared__ int32_t g_uids[ROUTED ? 64 : 1], g_urows[ROUTED ? 512 : 1], g_ucnt[ROUTED ? 64 : 1], g_nu[2];
   __shared__ float g_uw[ROUTED ? 512 : 1];
   __shared__ uint32_t g_gidx[ROUTED ? 64 : 1];
+  __shared__ __align__(16) uint32_t s_huge[4];
   const int u = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, i = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform (scalar registers)
@@ -267,33 +241,31 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) d
   wait_vm_all();   // the metadata loads are done; nothing the compiler tracks stays in flight past this point
   const GateupLds L = gateup_lds(a.H, rl);
   // the activation rows go first (they need only the metadata the weight addresses need as well)
-  constexpr int JMAX = ROUTED ? (HALF ? 5 : 3) : 9;   // routed batches stage at most 2 rows at once, others 8
-  stage_act_rows<JMAX, NW>(a, lds, L, 0, min(cnt, rl), tok, wave, lane);
+  constexpr int JMAX = ROUTED ? 4 : 8;  // routed batches stage at most 2 rows at once, others 4
+  stage_act_rows<JMAX>(a, lds, L, 0, min(cnt, rl), tok, wave, lane);
   __builtin_amdgcn_sched_barrier(0);
 
-  const int ntile = HALF ? 0 : (wave & 1), kr = HALF ? wave : (wave >> 1);
-  const int nb = blockIdx.x * BO;
-  const int n0 = nb + ntile * 16;
+  const int kr = wave;
+  const int n0 = blockIdx.x * 16;
   const size_t brow = (size_t)slot * a.I + n0 + i;
   const int ksplit = gateup_ksplit(a.H);
-  // with only two K-ranges (small H) waves 4-7 repeat K-range 0 and their partials are not used
+  // with only two K-ranges (small H) waves 2 and 3 repeat K-range 0 and their partials are not used
   const int k0 = (kr < ksplit ? kr : 0) * NS * 128;
   const int b0 = k0 / 32;
   const uint4* gw = reinterpret_cast<const uint4*>(a.gate_w + brow * (a.H / 8)) + b0 + g;   // one uint4 per 32-block
   const uint4* upw = reinterpret_cast<const uint4*>(a.up_w + brow * (a.H / 8)) + b0 + g;
-  // the block's gate and up scales (BO rows x H/32 bytes each, contiguous in the pools) in 8-byte pieces
-  constexpr int LG_BO = HALF ? 4 : 5;
+  // the block's gate and up scales (16 rows x H/32 bytes each, contiguous in the pools) in 8-byte pieces
   const int lg_pr = __builtin_ctz(a.H / 256);             // pieces per scale row = H / 256
-  const int npieces = (2 * BO) << lg_pr;
-  const int p0 = tid, p1 = tid + 64 * NW;
+  const int npieces = 32 << lg_pr;
+  const int p0 = tid, p1 = tid + 256;
   const int q0 = p0 < npieces ? p0 : 0, q1 = p1 < npieces ? p1 : 0;
   auto piece_src = [&](int p) {
-    const int proj = p >> (LG_BO + lg_pr), row = (p >> lg_pr) & (BO - 1), c = p & ((1 << lg_pr) - 1);
-    return reinterpret_cast<const uint2*>((proj ? a.up_s : a.gate_s) + ((size_t)slot * a.I + nb + row) * (a.H / 32)) + c;
+    const int proj = p >> (4 + lg_pr), row = (p >> lg_pr) & 15, c = p & ((1 << lg_pr) - 1);
+    return reinterpret_cast<const uint2*>((proj ? a.up_s : a.gate_s) + ((size_t)slot * a.I + n0 + row) * (a.H / 32)) + c;
   };
   auto piece_dst = [&](int p) {
-    const int proj = p >> (LG_BO + lg_pr), row = (p >> lg_pr) & (BO - 1), c = p & ((1 << lg_pr) - 1);
-    return reinterpret_cast<uint2*>(lds + (proj * 32 + row) * L.RS + 8 * c);
+    const int proj = p >> (4 + lg_pr), row = (p >> lg_pr) & 15, c = p & ((1 << lg_pr) - 1);
+    return reinterpret_cast<uint2*>(lds + (proj * 16 + row) * L.RS + 8 * c);
   };
   // the scale pieces, then the weight batch: the activation rows and the scales land first, so each MFMA step
   // can start as soon as its own weights arrive
@@ -319,70 +291,71 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) d
   wait_vm_keep<2 * NS>();    // everything before the weight batch has landed: staged rows and scale pieces
   if (p0 < npieces) *piece_dst(p0) = sp0;
   if (p1 < npieces) *piece_dst(p1) = sp1;
+  const uint64_t huge = __ballot(has_huge_scale(sp0) || has_huge_scale(sp1));
+  if (lane == 0) s_huge[wave] = huge != 0 ? 1u : 0u;
   __syncthreads();
+  uint32_t any_huge = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) any_huge |= s_huge[w];
+  const float fs = any_huge ? 0.25f : 1.0f;   // scale of the weights
 
   v4f accg = {0.0f, 0.0f, 0.0f, 0.0f}, accu = {0.0f, 0.0f, 0.0f, 0.0f};
-  const uint8_t* lrow = lds + (ntile * 16 + i) * L.RS + b0;   // this lane's gate scale row (up: + 32 rows)
-  const int crow = i & 7;              // the expert's row c carried by this lane (hi rows 0-7, lo rows 8-15)
-  // one pass over the staged rows: the operands of step s + 1 are read from LDS while step s multiplies
-  auto run_pass = [&](int c0) {
+  const uint8_t* lrow = lds + i * L.RS + b0;   // this lane's gate scale row (up: + 16 rows)
+  const int crow = i & 7;              // the expert's row c in this lane's column
+  // one pass over the staged rows: each activation operand of step s + 1 is read from LDS as step s is done with it
+  auto run_pass = [&](int c0, v4f oldg, v4f oldu) __attribute__((always_inline)) {
     const bool avalid = crow >= c0 && crow < min(cnt, c0 + rl);
-    const int lr = avalid ? crow - c0 : 0;
-    const uint8_t* arow_p = lds + (i < 8 ? L.a_hi : L.a_lo) + lr * L.RA + k0 + 16 * g;
-    const uint8_t* asc_p = lds + L.a_sc + lr * 2 * (a.H / 32) + (i < 8 ? 0 : a.H / 32) + b0;
-    uint4 p = *reinterpret_cast<const uint4*>(arow_p), q = *reinterpret_cast<const uint4*>(arow_p + 64);
-    uint32_t sw = *reinterpret_cast<const uint32_t*>(asc_p);
-    uint32_t gs = *reinterpret_cast<const uint32_t*>(lrow), us = *reinterpret_cast<const uint32_t*>(lrow + 32 * L.RS);
+    const uint8_t* xp = lds + L.act + (avalid ? crow - c0 : 0) * L.RA + 2 * k0 + 64 * g;
+    bf16x8 x[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) x[m] = lds_bf16x8(xp + 16 * m);
+    uint32_t gs = *reinterpret_cast<const uint32_t*>(lrow), us = *reinterpret_cast<const uint32_t*>(lrow + 16 * L.RS);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const uint4 pc = zero_if(p, avalid), qc = zero_if(q, avalid);
-      const int sa = avalid ? (int)byte_of(sw, g) : 127;
-      const int sgc = (int)byte_of(gs, g), suc = (int)byte_of(us, g);
+      const float scg = e8m0_f32(byte_of(gs, g)) * fs, scu = e8m0_f32(byte_of(us, g)) * fs;
       if (s + 1 < NS) {
-        p = *reinterpret_cast<const uint4*>(arow_p + 128 * (s + 1));
-        q = *reinterpret_cast<const uint4*>(arow_p + 128 * (s + 1) + 64);
-        sw = *reinterpret_cast<const uint32_t*>(asc_p + 4 * (s + 1));
         gs = *reinterpret_cast<const uint32_t*>(lrow + 4 * (s + 1));
-        us = *reinterpret_cast<const uint32_t*>(lrow + 32 * L.RS + 4 * (s + 1));
+        us = *reinterpret_cast<const uint32_t*>(lrow + 16 * L.RS + 4 * (s + 1));
       }
-      v8i A = {(int)pc.x, (int)pc.y, (int)pc.z, (int)pc.w, (int)qc.x, (int)qc.y, (int)qc.z, (int)qc.w};
-      accg = MFMA_F8xF4(A, b_operand(bg[s]), accg, sa, sgc);
-      accu = MFMA_F8xF4(A, b_operand(bu[s]), accu, sa, suc);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        accg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(bg[s], m), scg), x[m], accg, 0, 0, 0);
+        accu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(bu[s], m), scu), x[m], accu, 0, 0, 0);
+        if (s + 1 < NS) x[m] = lds_bf16x8(xp + 256 * (s + 1) + 16 * m);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {      // a column without a row of this pass keeps its sums
+      accg[q] = avalid ? accg[q] : oldg[q];
+      accu[q] = avalid ? accu[q] : oldu[q];
+    }
   };
-  run_pass(0);
+  run_pass(0, v4f{0.0f, 0.0f, 0.0f, 0.0f}, v4f{0.0f, 0.0f, 0.0f, 0.0f});
   for (int c0 = rl; c0 < cnt; c0 += rl) {   // rare: more rows routed to one expert than staged at once
     __syncthreads();
-    stage_act_rows<JMAX, NW>(a, lds, L, c0, min(cnt - c0, rl), tok, wave, lane);
+    stage_act_rows<JMAX>(a, lds, L, c0, min(cnt - c0, rl), tok, wave, lane);
     wait_vm_all();
     __syncthreads();
-    run_pass(c0);
+    run_pass(c0, accg, accu);
   }
-  mfma_f8f4_settle();
-  float vg[4], vu[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {   // rows 4g+q (hi, g < 2) plus rows 8+4g+q (lo) of lane l + 32
-    vg[q] = accg[q] + __shfl_xor(accg[q], 32, 64);
-    vu[q] = accu[q] + __shfl_xor(accu[q], 32, 64);
-  }
-  __syncthreads();                 // the activation region is free: K-range partials and the h tile go there
-  float (*red)[2][2][32][4] = reinterpret_cast<float (*)[2][2][32][4]>(lds + L.red);   // [K-range][ntile][g/u][lane][q]
-  float (*hl)[32] = reinterpret_cast<float (*)[32]>(lds + L.hl);
-  if (lane < 32) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) { red[kr][ntile][0][lane][q] = vg[q]; red[kr][ntile][1][lane][q] = vu[q]; }
+  accg = accg * (1.0f / fs);
+  accu = accu * (1.0f / fs);
+  __syncthreads();                 // the activation region is free: the K-range partials go there
+  float (*red)[2][32][4] = reinterpret_cast<float (*)[2][32][4]>(lds + L.red);   // [K-range][gate/up][8 g + row][q]
+  if (i < 8) {                     // lane (i, g): row i, outputs 4 g + q
+    *reinterpret_cast<v4f*>(red[kr][0][8 * g + i]) = accg;
+    *reinterpret_cast<v4f*>(red[kr][1][8 * g + i]) = accu;
   }
   __syncthreads();
   // SwiGLU, one (row, output) per thread: K-range partials summed in a fixed order (0, 1, 2, 3)
-  uint16_t hb = 0;
-  const int e_q = tid & 3, e_l = (tid >> 2) & 31, e_nt = HALF ? 0 : ((tid >> 7) & 1);
-  const int e_r = 4 * (e_l >> 4) + e_q, e_n = e_nt * 16 + (e_l & 15);
-  if (tid < 128 * NT) {
-    float gsum = red[0][e_nt][0][e_l][e_q], usum = red[0][e_nt][1][e_l][e_q];
+  if (tid < 128) {
+    const int e_r = tid >> 4, e_n = tid & 15;
+    const int e_l = 8 * (e_n >> 2) + e_r, e_q = e_n & 3;
+    float gsum = red[0][0][e_l][e_q], usum = red[0][1][e_l][e_q];
 #pragma unroll
     for (int j = 1; j < 4; ++j) {
-      const float pg = red[j][e_nt][0][e_l][e_q], pu = red[j][e_nt][1][e_l][e_q];
+      const float pg = red[j][0][e_l][e_q], pu = red[j][1][e_l][e_q];
       gsum += j < ksplit ? pg : 0.0f;
       usum += j < ksplit ? pu : 0.0f;
     }
@@ -390,42 +363,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) d
     const float gtf = bf16_to_f32(gt);
     const float ut = round_bf16(usum);
     const float sig = round_bf16(sigmoid_spec(gtf));   // the bf16 sigmoid table's entry for gt, computed in place
-    const float hv = round_bf16(round_bf16(gtf * sig) * ut);
-    hb = e_r < cnt ? f32_to_bf16(hv) : (uint16_t)0;
-    if constexpr (!HALF) hl[e_r][e_n] = e_r < cnt ? hv : 0.0f;
-  }
-  if constexpr (HALF) {            // h in bf16 for the down kernel's split (and the padding rows when asked)
-    if (tid < 128 && (e_r < cnt || (a.zero_pad && e_r < a.R)))
-      a.h[((size_t)u * a.R + e_r) * a.I + nb + e_n] = hb;
-    if (publisher) publish_routes(a, s_inds, s_w, g_uids, g_urows, g_ucnt, g_uw, g_gidx, g_nu, tid);
-    return;
-  }
-  __syncthreads();
-  if (a.zero_pad && tid < 256 && e_r < a.R)   // h itself only for callers that asked for the intermediates
-    a.h[((size_t)u * a.R + e_r) * a.I + nb + e_n] = hb;
-  if (tid < 256) {                 // hi/lo E4M3 split of h per (row, 32-block): one value per lane, a row per half-wave
-    const int r = tid >> 5, nl = tid & 31;
-    const float v = hl[r][nl];
-    // max over the 32 lanes of the row: DPP within each 16-lane row, then one exchange between the two rows
-    float amax = dpp_group_max16(fabsf(v));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    const int X = fp8_block_exp(amax);
-    float res;
-    const uint32_t hc = e4m3_encode(v, X, &res);
-    float ramax = dpp_group_max16(fabsf(res));
-    ramax = fmaxf(ramax, __shfl_xor(ramax, 16, 64));
-    const int Y = fp8_block_exp(ramax);
-    float lres;   // the lo code's own residual, unused
-    const uint32_t lc = e4m3_encode(res, Y, &lres);
-    if (r < cnt) {
-      const size_t row = (size_t)u * a.R + r;
-      a.hq_hi[row * a.I + nb + nl] = (uint8_t)hc;
-      a.hq_lo[row * a.I + nb + nl] = (uint8_t)lc;
-      if (nl == 0) {
-        a.hq_hs[row * (a.I / 32) + blockIdx.x] = (uint8_t)(X + 127);
-        a.hq_ls[row * (a.I / 32) + blockIdx.x] = (uint8_t)(Y + 127);
-      }
-    }
+    const uint16_t hb = f32_to_bf16(round_bf16(gtf * sig) * ut);
+    if (e_r < cnt || (a.zero_pad && e_r < a.R))   // padding rows (zeros) only for callers that asked for h
+      a.h[((size_t)u * a.R + e_r) * a.I + n0 + e_n] = e_r < cnt ? hb : (uint16_t)0;
   }
   if (publisher)   // block (0, 0) publishes the full routing for the down kernel
     publish_routes(a, s_inds, s_w, g_uids, g_urows, g_ucnt, g_uw, g_gidx, g_nu, tid);
@@ -442,29 +382,21 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) d
 // rounding of the gather_qmm path when asked, model.py:181), sums each row's k routes in route order
 // (kernels.py:198-199) and writes y.  No other block is waited for.
 
-// Per-wave LDS buffer of the down kernel for `rw` staged h rows of one K-half (KH = I / 2 codes):
-// hi rows (KH + 16 bytes each), lo rows (starting 128 bytes off the hi rows' bank phase), then per row the
-// [hi | lo] scales (2 x KH / 32 bytes).
+// Per-wave LDS buffer of the down kernel: `rw` staged bf16 h rows of one K-half (KH = I / 2), 2 KH + 16 bytes each.
 struct DownLds {
-  int KH, RA, hi, lo, sc, wave_bytes, part, total;
+  int KH, RA, wave_bytes, part, total;
 };
 __host__ __device__ inline DownLds down_lds(int I, int rw, int nroutes) {
   DownLds L;
   L.KH = I / 2;
-  L.RA = L.KH + 16;
-  L.hi = 0;
-  L.lo = align_up(rw * L.RA, 256) + 128;
-  L.sc = align_up(L.lo + rw * L.RA, 16);
-  L.wave_bytes = align_up(L.sc + rw * 2 * (L.KH / 32), 256);
+  L.RA = 2 * L.KH + 16;
+  L.wave_bytes = align_up(rw * L.RA, 256);
   L.part = 16 * L.wave_bytes;                       // [2][nroutes][16] floats
   L.total = L.part + 2 * nroutes * 16 * 4;
   return L;
 }
 
-// HSPLIT: h comes in bf16 (from the 16-output gate/up blocks) and each wave splits its item's rows into the hi/lo
-// E4M3 planes itself while its weights stream, a lane pair per 32-block and the (at most rw <= 2) staged rows one
-// after the other; the planes and scales are those the gate/up epilogue writes otherwise.
-template <int NS, bool HSPLIT = false>
+template <int NS>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) decode_down_combine_kernel(ExpertsArgs a, int rw) {
   extern __shared__ __align__(16) uint8_t dl[];
   __shared__ uint32_t cgidx[64];      // combine indices and weights, loaded with the routing metadata
@@ -495,54 +427,15 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     for (int b = 0; b < 4; ++b) prefv += __popcll(__ballot((c >> b) & 1) & below) << b;
   }
   uint8_t* wb = dl + wave * L.wave_bytes;
-  // h rows of the item staged at rows 0 .. n - 1 (n <= 3) of the wave's buffer: hi and lo codes of the K-half
-  // (KH <= 1024 bytes, one piece each) and the [hi | lo] scales
+  // h rows of the item staged at rows 0 .. n - 1 (n <= 3) of the wave's buffer: 2 KH <= 2048 bytes, one or two pieces
   auto stage = [&](int u, int kh, int c0, int n) {
-    const int sb = L.KH / 32;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       if (c >= n) break;
-      const size_t row = (size_t)u * a.R + c0 + c;
-      if (16 * lane < L.KH) {
-        lds_copy16(a.hq_hi + row * a.I + kh * L.KH, 16 * lane, wb + L.hi + c * L.RA);
-        lds_copy16(a.hq_lo + row * a.I + kh * L.KH, 16 * lane, wb + L.lo + c * L.RA);
-      }
-      const uint8_t* dst = wb + L.sc + c * 2 * sb;
-      if (4 * lane < sb) lds_copy4(a.hq_hs + row * (a.I / 32) + kh * sb, 4 * lane, dst);
-      else if (4 * lane < 2 * sb) lds_copy4(a.hq_ls + row * (a.I / 32) + kh * sb - sb, 4 * lane, dst);
-    }
-  };
-  // HSPLIT: lane l holds bf16 values 16 l .. 16 l + 15 of the K-half (block l / 2) of staged rows c0 and c0 + 1
-  auto hload = [&](int u, int kh, int c0, int n, bool active, uint4 (&hv)[2][2]) {
-    const bool live = active && 16 * lane < L.KH;
+      const uint16_t* row = a.h + ((size_t)u * a.R + c0 + c) * a.I + kh * L.KH;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const size_t row = (size_t)u * a.R + c0 + (c < n ? c : 0);
-      const uint4* hp = reinterpret_cast<const uint4*>(a.h + row * a.I + kh * L.KH + 16 * (live ? lane : 0));
-      hv[c][0] = hp[0];
-      hv[c][1] = hp[1];
-    }
-    return live;
-  };
-  // every lane calls this (the pair exchanges its block maxima); rows c < n of the live lanes are written
-  auto hsplit = [&](const uint4 (&hv)[2][2], int n, bool live) {
-    const int sb = L.KH / 32;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (c >= n) break;                            // wave-uniform
-      const uint32_t pw[8] = {hv[c][0].x, hv[c][0].y, hv[c][0].z, hv[c][0].w,
-                              hv[c][1].x, hv[c][1].y, hv[c][1].z, hv[c][1].w};
-      uint32_t hw[4], lw[4];
-      int X, Y;
-      quant_pair_fp8_hilo(pw, hw, lw, &X, &Y);
-      if (live) {
-        *reinterpret_cast<uint4*>(wb + L.hi + c * L.RA + 16 * lane) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-        *reinterpret_cast<uint4*>(wb + L.lo + c * L.RA + 16 * lane) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-        if ((lane & 1) == 0) {
-          wb[L.sc + c * 2 * sb + (lane >> 1)] = (uint8_t)(X + 127);
-          wb[L.sc + c * 2 * sb + sb + (lane >> 1)] = (uint8_t)(Y + 127);
-        }
-      }
+      for (int p = 0; p < 2; ++p)
+        if (1024 * p + 16 * lane < 2 * L.KH) lds_copy16(row + 512 * p, 16 * lane, wb + c * L.RA + 1024 * p);
     }
   };
   // scale staging: lane L loads 8 bytes of row L / LPR of the item's K-half (NS * 4 bytes per row)
@@ -556,10 +449,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     const int slot = __builtin_amdgcn_readlane(slotv, u);
     const int rbase = __builtin_amdgcn_readlane(prefv, u);
     const bool active = cnt > 0 && slot >= 0 && slot < a.S;
-    uint4 hv[2][2];
-    bool hlive = false;
-    if constexpr (HSPLIT) hlive = hload(u, kh, 0, min(cnt, rw), active, hv);
-    else if (active) stage(u, kh, 0, min(cnt, rw));
+    if (active) stage(u, kh, 0, min(cnt, rw));
     const int b0 = kh * NS * 4;      // first 32-block of this K-half
     const size_t bslot = (size_t)(active ? slot : 0) * a.H + m0;
     const uint4* dw = reinterpret_cast<const uint4*>(a.down_w + (bslot + i) * (a.I / 8)) + b0 + g;
@@ -570,66 +460,49 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     __builtin_amdgcn_sched_barrier(0);   // every weight load is in flight before anything waits
     wait_vm_keep<NS>();                  // the staged rows and the scales have landed; each MFMA step then waits
                                          // only for its own weights
-    if constexpr (HSPLIT) hsplit(hv, min(cnt, rw), hlive);   // while the weights stream
     if (lane < 16 * LPR) *reinterpret_cast<uint2*>(&wsc[wave][srow * SRS + 2 * spart]) = sraw;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t* srow_p = &wsc[wave][i * SRS];
-    // one pass over the staged rows: the operands of step s + 1 are read from LDS while step s multiplies
-    auto run_pass = [&](int c0) {
+    const float fs = __ballot(has_huge_scale(sraw)) ? 0.25f : 1.0f;
+    // one pass over the staged rows: each activation operand of step s + 1 is read from LDS as step s is done with it
+    auto run_pass = [&](int c0, v4f old) __attribute__((always_inline)) {
       const bool avalid = crow >= c0 && crow < min(cnt, c0 + rw);
-      const int lr = avalid ? crow - c0 : 0;
-      const uint8_t* arow_p = wb + (i < 8 ? L.hi : L.lo) + lr * L.RA + 16 * g;
-      const uint8_t* asc_p = wb + L.sc + lr * 2 * (L.KH / 32) + (i < 8 ? 0 : L.KH / 32);
-      uint4 p = *reinterpret_cast<const uint4*>(arow_p), q = *reinterpret_cast<const uint4*>(arow_p + 64);
-      uint32_t sw = *reinterpret_cast<const uint32_t*>(asc_p), bs = srow_p[0];
+      const uint8_t* xp = wb + (avalid ? crow - c0 : 0) * L.RA + 64 * g;
+      bf16x8 x[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) x[m] = lds_bf16x8(xp + 16 * m);
+      uint32_t bs = srow_p[0];
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        const uint4 pc = zero_if(p, avalid), qc = zero_if(q, avalid);
-        const int sa = avalid ? (int)byte_of(sw, g) : 127;
-        const int sb = (int)byte_of(bs, g);
-        if (s + 1 < NS) {
-          p = *reinterpret_cast<const uint4*>(arow_p + 128 * (s + 1));
-          q = *reinterpret_cast<const uint4*>(arow_p + 128 * (s + 1) + 64);
-          sw = *reinterpret_cast<const uint32_t*>(asc_p + 4 * (s + 1));
-          bs = srow_p[s + 1];
+        const float sc = e8m0_f32(byte_of(bs, g)) * fs;
+        if (s + 1 < NS) bs = srow_p[s + 1];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(bw[s], m), sc), x[m], acc, 0, 0, 0);
+          if (s + 1 < NS) x[m] = lds_bf16x8(xp + 256 * (s + 1) + 16 * m);
         }
-        v8i A = {(int)pc.x, (int)pc.y, (int)pc.z, (int)pc.w, (int)qc.x, (int)qc.y, (int)qc.z, (int)qc.w};
-        acc = MFMA_F8xF4(A, b_operand(bw[s]), acc, sa, sb);
         __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = avalid ? acc[q] : old[q];
     };
-    if (active) run_pass(0);
+    if (active) run_pass(0, v4f{0.0f, 0.0f, 0.0f, 0.0f});
     for (int c0 = rw; active && c0 < cnt; c0 += rw) {   // rare: more rows on one expert than the buffer holds
       __builtin_amdgcn_wave_barrier();
-      if constexpr (HSPLIT) {
-        uint4 hv2[2][2];
-        const bool live2 = hload(u, kh, c0, min(cnt - c0, rw), true, hv2);
-        wait_vm_all();
-        hsplit(hv2, min(cnt - c0, rw), live2);
-      } else {
-        stage(u, kh, c0, min(cnt - c0, rw));
-      }
+      stage(u, kh, c0, min(cnt - c0, rw));
       wait_vm_all();
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      run_pass(c0);
+      run_pass(c0, acc);
     }
+    acc = acc * (1.0f / fs);
     __builtin_amdgcn_wave_barrier();     // the staged rows and scales are read before the next item overwrites them
-    mfma_f8f4_settle();
-    float dq[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) dq[q] = acc[q] + __shfl_xor(acc[q], 32, 64);   // hi rows + lo rows
-    if (lane < 32) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = 4 * g + q;
-        if (r < cnt && rbase + r < nr) part[(kh * nr + rbase + r) * 16 + i] = dq[q];
-      }
-    }
+    if (i < cnt && i < 8 && rbase + i < nr)                      // lane (i, g): row i, outputs 4 g ..
+      *reinterpret_cast<v4f*>(&part[(kh * nr + rbase + i) * 16 + 4 * g]) = acc;
   }
   if (tid < nr) cgidx[tid] = gi;
   if (tid < UR) cuw[tid] = wi;
@@ -680,25 +553,15 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
 
 // ------------------------------------------------------------------ host
 struct ExpertsWs {
-  uint8_t *xq_hi, *xq_lo, *xq_hs, *xq_ls;
-  uint16_t* h;
-  uint8_t *hq_hi, *hq_lo, *hq_hs, *hq_ls;
+  uint16_t *r, *h;
   float* part;
 };
-// intermediates: room for the bf16 h and the fp32 partials, written only when a caller of mimo_moe_experts asks
-// for them (the fused decode never does); bf16_h: room for h alone (the two-row fused decode passes h in bf16)
-static ExpertsWs carve_experts(Carve& c, int M, int Umax, int R, int H, int I, bool intermediates,
-                               bool bf16_h = false) {
+// intermediates: room for the fp32 partials, written only when a caller of mimo_moe_experts asks for them (the fused
+// decode never does); rows: room for the normalised rows of a decoder-layer step
+static ExpertsWs carve_experts(Carve& c, int M, int Umax, int R, int H, int I, bool intermediates, bool rows) {
   ExpertsWs w{};
-  w.xq_hi = c.take<uint8_t>((size_t)M * H);
-  w.xq_lo = c.take<uint8_t>((size_t)M * H);
-  w.xq_hs = c.take<uint8_t>((size_t)M * H / 32);
-  w.xq_ls = c.take<uint8_t>((size_t)M * H / 32);
-  if (intermediates || bf16_h) w.h = c.take<uint16_t>((size_t)Umax * R * I);
-  w.hq_hi = c.take<uint8_t>((size_t)Umax * R * I);
-  w.hq_lo = c.take<uint8_t>((size_t)Umax * R * I);
-  w.hq_hs = c.take<uint8_t>((size_t)Umax * R * I / 32);
-  w.hq_ls = c.take<uint8_t>((size_t)Umax * R * I / 32);
+  if (rows) w.r = c.take<uint16_t>((size_t)M * H);
+  w.h = c.take<uint16_t>((size_t)Umax * R * I);
   if (intermediates) w.part = c.take<float>((size_t)Umax * R * H);
   return w;
 }
@@ -740,28 +603,17 @@ static int launch_gateup(const ExpertsArgs& a, int rl, hipStream_t st) {
   const size_t lds = (size_t)gateup_lds(a.H, rl).total;
   int rc = allow_lds(reinterpret_cast<const void*>(&decode_gateup_kernel<NS, ROUTED, FAST2>), lds, &allowed);
   if (rc) return rc;
-  decode_gateup_kernel<NS, ROUTED, FAST2><<<dim3(a.I / 32, a.Umax), 512, lds, st>>>(a, rl);
+  decode_gateup_kernel<NS, ROUTED, FAST2><<<dim3(a.I / 16, a.Umax), 256, lds, st>>>(a, rl);
   return MIMO_OK;
 }
 
-template <int NS, bool HSPLIT = false>
+template <int NS>
 static int launch_down(const ExpertsArgs& a, int rw, hipStream_t st) {
   static std::atomic<int> allowed{0};
   const size_t lds = (size_t)down_lds(a.I, rw, a.M * a.k).total;
-  int rc = allow_lds(reinterpret_cast<const void*>(&decode_down_combine_kernel<NS, HSPLIT>), lds, &allowed);
+  int rc = allow_lds(reinterpret_cast<const void*>(&decode_down_combine_kernel<NS>), lds, &allowed);
   if (rc) return rc;
-  decode_down_combine_kernel<NS, HSPLIT><<<a.H / 16, 1024, lds, st>>>(a, rw);
-  return MIMO_OK;
-}
-
-// one or two rows, expert ids as slots: 16-output gate/up blocks (h in bf16), the down kernel splitting h
-template <int NS, bool FAST2>
-static int launch_gateup_half(const ExpertsArgs& a, int rl, hipStream_t st) {
-  static std::atomic<int> allowed{0};
-  const size_t lds = (size_t)gateup_lds(a.H, rl).total;
-  int rc = allow_lds(reinterpret_cast<const void*>(&decode_gateup_kernel<NS, true, FAST2, true>), lds, &allowed);
-  if (rc) return rc;
-  decode_gateup_kernel<NS, true, FAST2, true><<<dim3(a.I / 16, a.Umax), 256, lds, st>>>(a, rl);
+  decode_down_combine_kernel<NS><<<a.H / 16, 1024, lds, st>>>(a, rw);
   return MIMO_OK;
 }
 
@@ -769,10 +621,10 @@ static int run_experts(const ExpertsArgs& base, int M, int round_bf16, hipStream
   ExpertsArgs a = base;
   a.round_bf16 = round_bf16;
   const int ns = gateup_steps(a.H);    // MFMA steps per wave
-  // activation rows staged at once: a row picks an expert at most once, so an expert gets at most M rows;
-  // more (a slot table mapping two experts of a row to one slot) costs extra passes, not wrong results
+  // activation rows staged at once (an expert with more takes extra passes): 4 keep a block's LDS within a quarter of
+  // the CU's, and few experts of a step have more; the routed kernel's own LDS leaves room for 2
   const bool fused_select = a.scores && a.Umax <= 16 && a.E <= 256;   // small batches: every block selects
-  const int rl = min(a.R, fused_select ? min(M, 2) : M);   // the routed kernel stages at most 2 rows at once
+  const int rl = min(a.R, fused_select ? min(M, 2) : min(M, 4));
   const int rw = min(min(a.R, M), 3);
   if (a.scores && !fused_select) {
     int rc = launch_select_group(a.scores, a.keys, a.M, a.E, a.k, a.slot_of, a.R, a.S, a.Umax, a.inds_out, a.w_out,
@@ -780,26 +632,12 @@ static int run_experts(const ExpertsArgs& base, int M, int round_bf16, hipStream
     if (rc) return rc;
   }
   int rc;
-  bool half = false;   // 16-output gate/up blocks, h split by the down kernel
   {
     ProfScope p(st, "decode_gateup");
     // two rows with expert ids as slots (E <= 256 for a fused selection): each block finds its own expert from
     // the two threshold searches alone (one row does the same inside the general routed kernel)
     const bool fast2 = fused_select && a.slot_of == nullptr && a.S >= a.E && M == 2;
-    const bool fast1 = fused_select && a.slot_of == nullptr && a.S >= a.E && M == 1;
-    half = (fast1 || fast2) && a.h != nullptr && rw <= 2 && !a.zero_pad;
-    if (half) {
-      switch (ns * 2 + (fast2 ? 1 : 0)) {
-        case 17: rc = launch_gateup_half<8, true>(a, rl, st); break;
-        case 16: rc = launch_gateup_half<8, false>(a, rl, st); break;
-        case 9: rc = launch_gateup_half<4, true>(a, rl, st); break;
-        case 8: rc = launch_gateup_half<4, false>(a, rl, st); break;
-        case 5: rc = launch_gateup_half<2, true>(a, rl, st); break;
-        case 4: rc = launch_gateup_half<2, false>(a, rl, st); break;
-        case 3: rc = launch_gateup_half<1, true>(a, rl, st); break;
-        default: rc = launch_gateup_half<1, false>(a, rl, st); break;
-      }
-    } else if (fused_select) {   // cheaper than a separate selection launch
+    if (fused_select) {   // cheaper than a separate selection launch
       switch (ns * 2 + (fast2 ? 1 : 0)) {
         case 17: rc = launch_gateup<8, true, true>(a, rl, st); break;
         case 16: rc = launch_gateup<8, true, false>(a, rl, st); break;
@@ -822,10 +660,7 @@ static int run_experts(const ExpertsArgs& base, int M, int round_bf16, hipStream
   if (rc) return rc;
   {
     ProfScope p(st, "decode_down_combine");
-    switch (a.I / 256 + (half ? 16 : 0)) {
-      case 24: rc = launch_down<8, true>(a, rw, st); break;
-      case 20: rc = launch_down<4, true>(a, rw, st); break;
-      case 18: rc = launch_down<2, true>(a, rw, st); break;
+    switch (a.I / 256) {
       case 8: rc = launch_down<8>(a, rw, st); break;
       case 4: rc = launch_down<4>(a, rw, st); break;
       default: rc = launch_down<2>(a, rw, st); break;
@@ -843,7 +678,7 @@ extern "C" {
 
 size_t mimo_moe_experts_workspace_size(int M, int Umax, int R, int H, int I) {
   Carve c(nullptr, 0);
-  carve_experts(c, M, Umax, R, H, I, true);
+  carve_experts(c, M, Umax, R, H, I, true, false);
   return c.off;
 }
 
@@ -863,19 +698,16 @@ int mimo_moe_experts(const uint16_t* x, int M, const mimo_bank* bank, const int3
                "moe_experts: x, y, part_out must be 16-byte aligned");
   const int H = bank->hidden, I = bank->inter;
   Carve c(ws, ws_bytes);
-  ExpertsWs w = carve_experts(c, M, Umax, R, H, I, true);
+  ExpertsWs w = carve_experts(c, M, Umax, R, H, I, true, false);
   MIMO_REQUIRE(ws && c.fits(), MIMO_ERR_WORKSPACE, "moe_experts: workspace too small (need %zu)", c.off);
   hipStream_t st = as_stream(stream);
-  rc = launch_quantize_fp8_hilo(x, M, H, w.xq_hi, w.xq_hs, w.xq_lo, w.xq_ls, st);
-  if (rc) return rc;
   ExpertsArgs a{};
-  a.xq_hi = w.xq_hi; a.xq_lo = w.xq_lo; a.xq_hs = w.xq_hs; a.xq_ls = w.xq_ls;
+  a.x = x;
   a.gate_w = bank->gate_w; a.up_w = bank->up_w; a.down_w = bank->down_w;
   a.gate_s = bank->gate_s; a.up_s = bank->up_s; a.down_s = bank->down_s;
   a.H = H; a.I = I; a.R = R; a.Umax = Umax; a.k = k; a.M = M; a.S = bank->n_slots;
   a.uslot = uslot; a.urows = urows; a.ucnt = ucnt; a.n_unique = n_unique; a.uw = uw; a.gidx = gidx;
   a.h = h_out ? h_out : w.h;
-  a.hq_hi = w.hq_hi; a.hq_lo = w.hq_lo; a.hq_hs = w.hq_hs; a.hq_ls = w.hq_ls;
   a.part = part_out ? part_out : w.part;
   a.zero_pad = (h_out || part_out) ? 1 : 0;
   a.y = y;
@@ -910,14 +742,14 @@ size_t mimo_moe_decode_workspace_size(int M, int E, int k, int H, int I) {
   int32_t *inds, *uids, *urows, *ucnt, *nu, *st;
   uint32_t* gidx;
   carve_decode(c, M, E, k, Umax, kDecodeR, &l, &s, &kk, &inds, &w, &uids, &urows, &ucnt, &uw, &gidx, &nu, &st);
-  carve_experts(c, M, Umax, kDecodeR, H, I, false, M <= 2);
+  carve_experts(c, M, Umax, kDecodeR, H, I, false, true);
   return c.off;
 }
 
 }  // extern "C"
 
 namespace mimo {
-// The fused decode block on rows x (router logits + hi/lo split, experts, combine); resid: optional residual
+// The fused decode block on rows x (router logits, experts, combine); resid: optional residual
 // stream added in the combine; norm_w: optional RMSNorm of the rows inside the router kernel (r to r_out if given).
 static int decode_impl(const uint16_t* x, int M, const uint16_t* Wg, const float* bias, const int32_t* slot_of, int E,
                        int k, const mimo_bank* bank, uint16_t* y, int32_t* inds_out, float* w_out,
@@ -938,24 +770,23 @@ static int decode_impl(const uint16_t* x, int M, const uint16_t* Wg, const float
   uint32_t* gidx;
   carve_decode(c, M, E, k, Umax, kDecodeR, &logits, &scores, &keys, &inds, &w, &uids, &urows, &ucnt, &uw,
                &gidx, &nu, &status);
-  ExpertsWs ew = carve_experts(c, M, Umax, kDecodeR, H, I, false, M <= 2);
+  ExpertsWs ew = carve_experts(c, M, Umax, kDecodeR, H, I, false, true);
   MIMO_REQUIRE(ws && c.fits(), MIMO_ERR_WORKSPACE, "moe_decode: workspace too small (need %zu)", c.off);
 
   RouterSmallArgs ra{};
   ra.x = x; ra.Wg = Wg; ra.bias = bias; ra.T = M; ra.H = H; ra.E = E; ra.k = k;
   ra.logits = logits; ra.scores = scores; ra.keys = keys;
-  ra.xq_hi = ew.xq_hi; ra.xq_lo = ew.xq_lo; ra.xq_hs = ew.xq_hs; ra.xq_ls = ew.xq_ls;
-  ra.norm_w = norm_w; ra.eps = eps; ra.r_out = r_out;
+  ra.norm_w = norm_w; ra.eps = eps; ra.r_out = norm_w ? (r_out ? r_out : ew.r) : nullptr;
   rc = launch_router_logits_small(ra, st);
   if (rc) return rc;
 
   ExpertsArgs a{};
-  a.xq_hi = ew.xq_hi; a.xq_lo = ew.xq_lo; a.xq_hs = ew.xq_hs; a.xq_ls = ew.xq_ls;
+  a.x = norm_w ? ra.r_out : x;
   a.gate_w = bank->gate_w; a.up_w = bank->up_w; a.down_w = bank->down_w;
   a.gate_s = bank->gate_s; a.up_s = bank->up_s; a.down_s = bank->down_s;
   a.H = H; a.I = I; a.R = kDecodeR; a.Umax = Umax; a.k = k; a.M = M; a.S = S;
   a.uslot = uids; a.urows = urows; a.ucnt = ucnt; a.n_unique = nu; a.uw = uw; a.gidx = gidx;
-  a.h = ew.h; a.hq_hi = ew.hq_hi; a.hq_lo = ew.hq_lo; a.hq_hs = ew.hq_hs; a.hq_ls = ew.hq_ls;
+  a.h = ew.h;
   a.part = ew.part; a.zero_pad = 0; a.y = y;
   a.scores = scores; a.keys = keys; a.E = E; a.slot_of = slot_of;
   a.inds_out = inds_out ? inds_out : inds;
@@ -978,8 +809,7 @@ int mimo_moe_decode(const uint16_t* x, int M, const uint16_t* Wg, const float* b
                      status_out, ws, ws_bytes, as_stream(stream));
 }
 
-// The layer step normalises the rows inside the router kernel: no rows of r are kept unless r_out asks for them,
-// so the workspace is the decode block's.
+// The layer step normalises the rows inside the router kernel; the workspace has room for them in both steps.
 size_t mimo_moe_layer_decode_workspace_size(int M, int E, int k, int H, int I) {
   return mimo_moe_decode_workspace_size(M, E, k, H, I);
 }

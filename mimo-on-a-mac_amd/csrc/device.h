@@ -8,6 +8,8 @@ namespace mimo {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // ------------------------------------------------------------------ bf16
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -34,27 +36,19 @@ __device__ __forceinline__ uint32_t e2m1_mag_code(float y) {
   return (uint32_t)(v * 2.0f);  // 0, 1, 2, 3
 }
 
+// Eight E2M1 codes (low nibble first) times the power of two of `scale`: exact in bf16 for every scale byte up to 252
+// (checked on MI355X for every code; the conversion reads the scale's exponent field alone, so byte 0 is 2^-127 and
+// byte 255 gives NaN).  Bytes 253 and 254 make weights of 2^128 and more, which bf16 cannot hold.
+__device__ __forceinline__ bf16x8 fp4_bf16x8(uint32_t w, float scale) {
+  const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0);
+  const bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1);
+  const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2);
+  const bf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3);
+  return bf16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+__device__ __forceinline__ float e8m0_f32(uint32_t byte) { return __uint_as_float(byte << 23); }
+
 // ------------------------------------------------------------------ E4M3 (activation hi/lo split)
-// magnitude code for 0 <= y <= 448 (y exactly representable scaling of a bf16 value), nearest-even.
-__device__ __forceinline__ uint32_t e4m3_mag_code(float y) {
-  // below 2^-6: subnormal, quantum 2^-9 (a result of 8 is the smallest normal, same encoding)
-  const uint32_t sub = (uint32_t)rintf(y * 512.0f);
-  const uint32_t u = __float_as_uint(y);
-  int e = (int)((u >> 23) & 0xFF) - 127;
-  const uint32_t f = u & 0x7FFFFFu;
-  uint32_t q = f >> 20;
-  const uint32_t rem = f & 0xFFFFFu;
-  q += (rem > 0x80000u || (rem == 0x80000u && (q & 1u))) ? 1u : 0u;
-  e += q == 8u ? 1 : 0;
-  q = q == 8u ? 0u : q;
-  uint32_t code = ((uint32_t)(e + 7) << 3) | q;
-  code = code > 0x7Eu ? 0x7Eu : code;
-  return y < 0.015625f ? sub : code;
-}
-__device__ __forceinline__ float e4m3_decode_mag(uint32_t c) {
-  uint32_t e = (c >> 3) & 0xF, m = c & 7;
-  return e == 0 ? (float)m * 0.001953125f : __uint_as_float(((e + 120u) << 23) | (m << 20));
-}
 // E8M0 exponent X for an E4M3 block with maximum magnitude amax: amax / 2^X in (224, 448].
 __device__ __forceinline__ int fp8_block_exp(float amax) {
   if (amax == 0.0f) return 0;
@@ -67,26 +61,9 @@ __device__ __forceinline__ int fp8_block_exp(float amax) {
 __device__ __forceinline__ float exp2i(int X) {   // 2^X for -127 <= X <= 127, exact
   return X >= -126 ? __uint_as_float((uint32_t)(X + 127) << 23) : __uint_as_float(0x00400000u);
 }
-// Signed E4M3 code of v / 2^X (positive zero for a zero magnitude); writes the residual v - code * 2^X, computed
-// as one fused multiply-add: the difference is exact and the product, which can pass the fp32 range for the
-// largest blocks (448 * 2^120), is never rounded on its own.
-// A non-finite v (NaN or +-inf; E4M3 has no infinity) gets the E4M3 NaN code 0x7F and a NaN residual, as the
-// hardware conversion gives, so every product of its row is NaN.
-__device__ __forceinline__ uint32_t e4m3_encode(float v, int X, float* res) {
-  float inv = exp2i(-X);        // exact when -X in range; X >= -127 so -X <= 127
-  float y = fabsf(v) * inv;
-  uint32_t mag = e4m3_mag_code(y);
-  float dm = e4m3_decode_mag(mag);
-  uint32_t sgn = (mag != 0u && v < 0.0f) ? 0x80u : 0u;
-  const bool finite = fabsf(v) <= 3.40282347e38f;
-  const float r = __builtin_fmaf(sgn ? dm : -dm, exp2i(X), v);
-  *res = finite ? r : __uint_as_float(0x7FC00000u);
-  return finite ? (mag | sgn) : 0x7Fu;
-}
-
 // Two E4M3 codes (bits 0-7 and 8-15) of values already divided by their block scale (|y| <= 448) from the
-// hardware conversion (OCP E4M3, round to nearest even, checked against the oracle on every bf16 input), with
-// the sign of zero codes cleared: the codes e4m3_encode gives.
+// hardware conversion (OCP E4M3, round to nearest even, checked against the oracle on every bf16 input; a NaN or an
+// infinity gives the E4M3 NaN), with the sign of zero codes cleared.
 __device__ __forceinline__ uint32_t e4m3_pack2(float y0, float y1) {
   const uint32_t w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, 0, false) & 0xFFFFu;
   const uint32_t t = w & 0x7F7Fu;
@@ -138,7 +115,7 @@ __device__ __forceinline__ float sigmoid_spec(float xf) {
 
 // 32 bf16-valued floats -> hi / lo E4M3 words (4 codes per word, element order) and E8M0 bytes: hi = E4M3 block
 // quantisation of v, lo = the same of the exact residual v - hi.  Codes from the hardware conversion
-// (v_cvt_pk_fp8_f32: OCP E4M3, round to nearest even, checked against e4m3_encode on every bf16 input;
+// (v_cvt_pk_fp8_f32: OCP E4M3, round to nearest even, checked against the oracle on every bf16 input;
 // e4m3_pack2 clears the sign of zero codes); the scalings by 2^-X and 2^-Y are exact, and the residual is one
 // fused multiply-add (exact, with no overflow of the product for the largest blocks).
 __device__ __forceinline__ void quant_block_fp8_hilo(const float* v, uint32_t* hw, uint32_t* lw, uint8_t* hsb,
@@ -172,49 +149,6 @@ __device__ __forceinline__ void quant_block_fp8_hilo(const float* v, uint32_t* h
   *lsb = (uint8_t)(Y + 127);
 }
 
-// The same split of a 32-value block held by two adjacent lanes (lane pair l, l ^ 1: values 16 (l & 1) .. of the
-// block), 16 bf16 values per lane packed two per word (element 2 j in the low half of p[j]).  Every lane of the
-// wave calls it (the block maxima are exchanged between the pair); per element the operations are those of
-// quant_block_fp8_hilo, so the codes and exponents are the same.  hw, lw: 4 words of codes each; X, Y: the
-// block's hi and lo exponents (E8M0 byte = exponent + 127).
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-__device__ __forceinline__ void quant_pair_fp8_hilo(const uint32_t (&p)[8], uint32_t (&hw)[4], uint32_t (&lw)[4],
-                                                    int* Xo, int* Yo) {
-  float amax = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fmaxf(fabsf(bf16_lo(p[j])), fabsf(bf16_hi(p[j]))));
-  amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
-  const int X = fp8_block_exp(amax);
-  const float sx = exp2i(-X), dx = exp2i(X);
-  float ramax = 0.0f;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float v0 = bf16_lo(p[2 * w]), v1 = bf16_hi(p[2 * w]), v2 = bf16_lo(p[2 * w + 1]), v3 = bf16_hi(p[2 * w + 1]);
-    const uint32_t c01 = e4m3_pack2(v0 * sx, v1 * sx);
-    const uint32_t c23 = e4m3_pack2(v2 * sx, v3 * sx);
-    hw[w] = c01 | (c23 << 16);
-    const v2f d01 = e4m3_unpack2(c01), d23 = e4m3_unpack2(c23);
-    ramax = fmaxf(ramax, fabsf(__builtin_fmaf(-d01.x, dx, v0)));
-    ramax = fmaxf(ramax, fabsf(__builtin_fmaf(-d01.y, dx, v1)));
-    ramax = fmaxf(ramax, fabsf(__builtin_fmaf(-d23.x, dx, v2)));
-    ramax = fmaxf(ramax, fabsf(__builtin_fmaf(-d23.y, dx, v3)));
-  }
-  ramax = fmaxf(ramax, __shfl_xor(ramax, 1, 64));
-  const int Y = fp8_block_exp(ramax);
-  const float sy = exp2i(-Y);
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float v0 = bf16_lo(p[2 * w]), v1 = bf16_hi(p[2 * w]), v2 = bf16_lo(p[2 * w + 1]), v3 = bf16_hi(p[2 * w + 1]);
-    const v2f d01 = e4m3_unpack2(hw[w] & 0xFFFFu), d23 = e4m3_unpack2(hw[w] >> 16);
-    const float r0 = __builtin_fmaf(-d01.x, dx, v0), r1 = __builtin_fmaf(-d01.y, dx, v1);
-    const float r2 = __builtin_fmaf(-d23.x, dx, v2), r3 = __builtin_fmaf(-d23.y, dx, v3);
-    lw[w] = e4m3_pack2(r0 * sy, r1 * sy) | (e4m3_pack2(r2 * sy, r3 * sy) << 16);
-  }
-  *Xo = X;
-  *Yo = Y;
-}
-
 // ------------------------------------------------------------------ wave reductions (wave64)
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -237,21 +171,6 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
 // max over groups of `width` consecutive lanes (width a power of two <= 64)
 __device__ __forceinline__ float group_max(float v, int width) {
   for (int o = width >> 1; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-// max over each group of 8 consecutive lanes through DPP (xor 1, xor 2 within quads, then the half-row mirror)
-__device__ __forceinline__ float dpp_group_max8(float v) {
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0xB1, 0xF, 0xF, false)));
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x4E, 0xF, 0xF, false)));
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x141, 0xF, 0xF, false)));
-  return v;
-}
-
-// max over each group of 16 consecutive lanes (a DPP row): the 8-lane steps, then the row mirror
-__device__ __forceinline__ float dpp_group_max16(float v) {
-  v = dpp_group_max8(v);
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x140, 0xF, 0xF, false)));
   return v;
 }
 
@@ -341,22 +260,11 @@ __device__ __forceinline__ void gload16(v4i& dst, const void* gbase, uint32_t vo
 __device__ __forceinline__ void wait_vm_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 // s_waitcnt vmcnt(N): at most the N most recent vector memory loads still in flight (loads, including the LDS
 // copies above, complete in issue order, so everything issued before them has landed)
+__host__ __device__ constexpr int vm_keep(int n) { return (n & 15) | (7 << 4) | (15 << 8) | (((n >> 4) & 3) << 14); }
 template <int N>
 __device__ __forceinline__ void wait_vm_keep() {
   static_assert(N >= 0 && N < 64, "vmcnt holds 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | (((N >> 4) & 3) << 14));
-}
-
-// ------------------------------------------------------------------ MFMA result reads
-// The block-scaled fp8 x fp4 MFMA (v_mfma_scale_f32_16x16x128_f8f6f4 with an E4M3 A operand) runs 16 passes, but
-// the compiler pads a read of its result as if it took fewer: an epilogue that read the accumulator 12 wait
-// states after the last MFMA got values the MFMA had not finished writing (found on MI355X in a kernel whose
-// second MFMA was followed by a short epilogue).  Placed after a chain of these MFMAs and before anything reads
-// the accumulators, this waits 20 states and keeps the scheduler from moving instructions across it.
-__device__ __forceinline__ void mfma_f8f4_settle() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(vm_keep(N));
 }
 
 // ------------------------------------------------------------------ misc

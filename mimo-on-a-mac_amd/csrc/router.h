@@ -13,15 +13,14 @@ struct RouterSmallArgs {
   float* logits;           // [T, E]
   float* scores;           // [T, E] sigmoid (optional)
   float* keys;             // [T, E] sigmoid + bias (optional)
-  uint8_t *xq_hi, *xq_lo, *xq_hs, *xq_ls;   // optional fp8 split of x: [T, H], [T, H/32]
-  // optional RMSNorm of the rows first (the post-attention norm of a decoder layer): logits and split are then of
+  // optional RMSNorm of the rows first (the post-attention norm of a decoder layer): the logits are then of
   // r = RMSNorm(x) * norm_w, and r itself goes to r_out when given (H a multiple of 256)
   const uint16_t* norm_w;  // [H] bf16
   float eps;
   uint16_t* r_out;         // [T, H] bf16 (optional)
 };
 
-int launch_router_logits_small(const RouterSmallArgs& a, hipStream_t st);   // logits, sigmoid, keys, x split
+int launch_router_logits_small(const RouterSmallArgs& a, hipStream_t st);   // logits, sigmoid, keys, normalised rows
 
 struct SelectGroupArgs {
   const float *scores, *keys;   // [T, E]
@@ -46,17 +45,15 @@ int launch_router_logits(const uint16_t* x, const uint16_t* W, int T, int H, int
 int launch_router_select(const float* logits, const float* bias, int T, int E, int k, float scaling, int32_t* inds,
                          float* w, const int32_t* slot_of, int32_t* slot_inds, int n_slots, int32_t* status,
                          hipStream_t st);
-// Row tiles of the grouped GEMM: a slot with 1..narrow_max routes is one narrow tile; a larger one is split into
-// ceil(count / wide_rows) wide tiles of near-equal whole unit-route chunks (wide_rows a multiple of unit).
+// Row tiles of the grouped GEMM: a slot with 1..narrow_max routes is one narrow tile; a larger one is cut into wide
+// tiles of wide_rows routes and one of the remainder.
 // tiles[0] = (wide count, narrow count), wide tile t at tiles[1 + t], narrow tile t at tiles[1 + wcap + t], each
 // (slot, first route, end route, 0).
 struct TileSpec {
-  int narrow_max, wide_rows, wcap, unit;
+  int narrow_max, wide_rows, wcap;
 };
 int launch_dispatch(const int32_t* slots, int n, int n_slots, int32_t* hist, int32_t* perm, int32_t* offsets,
-                    int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, hipStream_t st);
+                    int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, bool zero_status, hipStream_t st);
 size_t dispatch_workspace(int n, int n_slots);
-int launch_quantize_fp8_hilo(const uint16_t* x, int64_t rows, int64_t cols, uint8_t* hi, uint8_t* hs, uint8_t* lo,
-                             uint8_t* ls, hipStream_t st, int32_t* zero_status = nullptr);
 
 }  // namespace mimo

@@ -75,64 +75,41 @@ __device__ void block_group_routes(const int32_t* inds, const float* scores, con
 //  router_logits_small_kernel: blocks [0, nlog = E) give one block per expert: T logits (fp32 FMA over bf16
 //    products; each wave a quarter of the row, loaded in one batch with the T activation rows, summed through
 //    DPP and then in LDS in a fixed order), then sigmoid and key by one thread per row;
-//    blocks [nlog, ...) split x into hi/lo E4M3 halves for the expert kernels (one thread per 32-block).
+//    blocks [nlog, ...) write the normalised rows r when a decoder-layer step asks for the norm.
 //  router_select_group_kernel (one block): top-k per row (one wave per row) and the grouping by slot.
-template <int NCH>
-__global__ void __launch_bounds__(256) router_logits_small_kernel(RouterSmallArgs a) {
+// A block has four waves for every RT rows (groups of RT, the last may hold fewer).
+template <int NCH, int RT>
+__global__ void __launch_bounds__(1024) router_logits_small_kernel(RouterSmallArgs a) {
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);   // quarter of the row
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int r0 = RT * grp, nr = min(RT, a.T - r0);                            // the group's rows
   const int q4 = a.H / 4;
   const bool norm = a.norm_w != nullptr;
   __shared__ float wsum[8][4];            // per row, the 4 wave sums of squares (norm only)
-  if ((int)blockIdx.x >= a.nlog) {           // hi/lo split of x: one element per lane, 32 lanes per block
-    if (!a.xq_hi && !a.r_out) return;
-    const int64_t n = (int64_t)a.T * a.H;
-    const int64_t idx = ((int64_t)(blockIdx.x - a.nlog) * blockDim.x + threadIdx.x);
-    const bool live = idx < n;
-    uint16_t xb = live ? a.x[idx] : (uint16_t)0;
-    if (norm) {
-      // the block's 256 elements lie in one row (H a multiple of 256): that row's inverse RMS, computed exactly as
-      // the logits blocks and the norm kernel compute it
-      const int64_t row = ((int64_t)(blockIdx.x - a.nlog) * blockDim.x) / a.H;
-      const uint16_t wb = a.norm_w[live ? idx - row * a.H : 0];
-      const uint16_t* xq = a.x + row * a.H + wave * q4;
-      uint4 xv[NCH];
-      bool ok[NCH];
+  if ((int)blockIdx.x >= a.nlog) {           // r = RMSNorm(x) * norm_w, one element per thread
+    // a group's 256 elements lie in one row (H a multiple of 256): that row's inverse RMS, computed exactly as the
+    // logits blocks and the norm kernel compute it
+    const int64_t first = (int64_t)(blockIdx.x - a.nlog) * blockDim.x + 256 * grp, idx = first + (threadIdx.x & 255);
+    const bool live = first < (int64_t)a.T * a.H;
+    const int64_t row = live ? first / a.H : 0;
+    const uint16_t xb = a.x[live ? idx : 0], wb = a.norm_w[live ? idx - row * a.H : 0];
+    const uint16_t* xq = a.x + row * a.H + wave * q4;
+    uint4 xv[NCH];
+    bool ok[NCH];
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
-        const int off = c * 512 + lane * 8;
-        ok[c] = off < q4;
-        xv[c] = *reinterpret_cast<const uint4*>(xq + (ok[c] ? off : 0));
-      }
-      float ss = 0.0f;
+    for (int c = 0; c < NCH; ++c) {
+      const int off = c * 512 + lane * 8;
+      ok[c] = off < q4;
+      xv[c] = *reinterpret_cast<const uint4*>(xq + (ok[c] ? off : 0));
+    }
+    float ss = 0.0f;
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) ss = ok[c] ? norm_sq_add8(xv[c], ss) : ss;
-      ss = norm_wave_sum(ss);
-      if (lane == 0) wsum[0][wave] = ss;
-      __syncthreads();
-      xb = norm_apply1(xb, wb, norm_inv(wsum[0], a.H, a.eps));
-      if (live && a.r_out) a.r_out[idx] = xb;
-      if (!a.xq_hi) return;
-    }
-    const float v = live ? bf16_to_f32(xb) : 0.0f;
-    float amax = dpp_group_max16(fabsf(v));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    const int X = fp8_block_exp(amax);
-    float res;
-    const uint32_t hc = e4m3_encode(v, X, &res);
-    float ramax = dpp_group_max16(fabsf(res));
-    ramax = fmaxf(ramax, __shfl_xor(ramax, 16, 64));
-    const int Y = fp8_block_exp(ramax);
-    float lres;   // the lo code's own residual, unused
-    const uint32_t lc = e4m3_encode(res, Y, &lres);
-    if (live) {
-      a.xq_hi[idx] = (uint8_t)hc;
-      a.xq_lo[idx] = (uint8_t)lc;
-      if ((lane & 31) == 0) {
-        a.xq_hs[idx >> 5] = (uint8_t)(X + 127);
-        a.xq_ls[idx >> 5] = (uint8_t)(Y + 127);
-      }
-    }
+    for (int c = 0; c < NCH; ++c) ss = ok[c] ? norm_sq_add8(xv[c], ss) : ss;
+    ss = norm_wave_sum(ss);
+    if (lane == 0) wsum[grp][wave] = ss;
+    __syncthreads();
+    if (live) a.r_out[idx] = norm_apply1(xb, wb, norm_inv(wsum[grp], a.H, a.eps));
     return;
   }
   // block e: expert e's logits for the T <= 8 rows.  Wave w covers elements [w H/4, (w+1) H/4): lane owns the
@@ -140,7 +117,7 @@ __global__ void __launch_bounds__(256) router_logits_small_kernel(RouterSmallArg
   __shared__ float part[8][4];
   const int e = blockIdx.x;
   const uint16_t* wrow = a.Wg + (size_t)e * a.H + wave * q4;
-  uint4 wq[NCH], xq[8][NCH], nw[NCH];
+  uint4 wq[NCH], xq[RT][NCH], nw[NCH];
   bool ok[NCH];
   // the expert's selection bias comes in with the first batch: loaded after the logit stores below it would be
   // one more memory round trip at the end of every block (the compiler cannot move it above stores it may alias)
@@ -153,37 +130,37 @@ __global__ void __launch_bounds__(256) router_logits_small_kernel(RouterSmallArg
     if (norm) nw[c] = *reinterpret_cast<const uint4*>(a.norm_w + wave * q4 + (ok[c] ? off : 0));
   }
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const uint16_t* xrow = a.x + (size_t)(r < a.T ? r : 0) * a.H + wave * q4;
+  for (int r = 0; r < RT; ++r) {
+    const uint16_t* xrow = a.x + (size_t)(r < nr ? r0 + r : 0) * a.H + wave * q4;
 #pragma unroll
     for (int c = 0; c < NCH; ++c)
-      if (r < a.T) xq[r][c] = *reinterpret_cast<const uint4*>(xrow + (ok[c] ? c * 512 + lane * 8 : 0));
+      if (r < nr) xq[r][c] = *reinterpret_cast<const uint4*>(xrow + (ok[c] ? c * 512 + lane * 8 : 0));
   }
   __builtin_amdgcn_sched_barrier(0);     // every load is in flight before the arithmetic
   if (norm) {                            // rows -> r: sums of squares in the norm kernel's order, then r in place
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      if (r < a.T) {
+    for (int r = 0; r < RT; ++r) {
+      if (r < nr) {
         float ss = 0.0f;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) ss = ok[c] ? norm_sq_add8(xq[r][c], ss) : ss;
         ss = norm_wave_sum(ss);
-        if (lane == 0) wsum[r][wave] = ss;
+        if (lane == 0) wsum[r0 + r][wave] = ss;
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      if (r < a.T) {
-        const float inv = norm_inv(wsum[r], a.H, a.eps);
+    for (int r = 0; r < RT; ++r) {
+      if (r < nr) {
+        const float inv = norm_inv(wsum[r0 + r], a.H, a.eps);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) xq[r][c] = norm_apply8(xq[r][c], nw[c], inv);
       }
     }
   }
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    if (r < a.T) {
+  for (int r = 0; r < RT; ++r) {
+    if (r < nr) {
       float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // four independent chains, added in a fixed order
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
@@ -197,7 +174,7 @@ __global__ void __launch_bounds__(256) router_logits_small_kernel(RouterSmallArg
         }
       }
       const float s = dpp_sum_f32((acc[0] + acc[1]) + (acc[2] + acc[3]));
-      if (lane == 0) part[r][wave] = s;
+      if (lane == 0) part[r0 + r][wave] = s;
     }
   }
   __syncthreads();
@@ -432,13 +409,15 @@ __device__ __forceinline__ int checked_slot(const int32_t* slots, int i, int n_s
   return s;
 }
 
+// zero_status (optional): a status word cleared here, for the placement kernel queued after it to flag bad slots in
 __global__ void __launch_bounds__(1024) dispatch_hist_kernel(const int32_t* __restrict__ slots, int n, int n_slots,
-                                                             int32_t* __restrict__ hist, int32_t* status) {
+                                                             int32_t* __restrict__ hist, int32_t* zero_status) {
   extern __shared__ int h[];
+  if (zero_status && blockIdx.x == 0 && threadIdx.x == 0) *zero_status = 0;
   for (int i = threadIdx.x; i < n_slots; i += blockDim.x) h[i] = 0;
   __syncthreads();
   int i = blockIdx.x * DISPATCH_CHUNK + threadIdx.x;
-  if (i < n) atomicAdd(&h[checked_slot(slots, i, n_slots, status)], 1);   // integer counts: order independent
+  if (i < n) atomicAdd(&h[checked_slot(slots, i, n_slots, nullptr)], 1);   // integer counts: order independent
   __syncthreads();
   for (int s = threadIdx.x; s < n_slots; s += blockDim.x) hist[(size_t)blockIdx.x * n_slots + s] = h[s];
 }
@@ -452,7 +431,8 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
                                                                    const int32_t* __restrict__ hist, int nchunks,
                                                                    int n_slots, int32_t* __restrict__ offsets,
                                                                    TileSpec spec, int4* __restrict__ tiles,
-                                                                   int32_t* __restrict__ perm, int32_t* __restrict__ inv) {
+                                                                   int32_t* __restrict__ perm, int32_t* __restrict__ inv,
+                                                                   int32_t* status) {
   extern __shared__ int dsp[];                   // base[n_slots], then wc[16 waves][n_slots] (counts <= 64)
   int* base = dsp;
   uint16_t* wc = reinterpret_cast<uint16_t*>(dsp + n_slots);
@@ -507,19 +487,15 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
         if (tiles) tiles[0] = make_int4(v1, v2, 0, 0);
       }
       if (nw) {
-        const int chunks = (c + spec.unit - 1) / spec.unit;
-        for (int q = 0; q < nw; ++q) {
-          const int c0 = (int)((int64_t)q * chunks / nw), c1 = (int)((int64_t)(q + 1) * chunks / nw);
-          tiles[1 + e1 + q] = make_int4(tid, e0 + spec.unit * c0, e0 + min(spec.unit * c1, c), 0);
-        }
+        for (int q = 0; q < nw; ++q)
+          tiles[1 + e1 + q] = make_int4(tid, e0 + spec.wide_rows * q, e0 + min(spec.wide_rows * (q + 1), c), 0);
       }
       if (ns) tiles[1 + spec.wcap + e2] = make_int4(tid, e0, e0 + c, 0);
     }
   }
-  // placement of this chunk's routes (slot ids were range-checked and flagged by dispatch_hist_kernel; clamped
-  // identically here)
+  // placement of this chunk's routes (slot ids clamped as dispatch_hist_kernel counted them, bad ones flagged)
   const int i = blk * DISPATCH_CHUNK + tid;
-  const int sl = i < n ? checked_slot(slots, i, n_slots, nullptr) : -1;
+  const int sl = i < n ? checked_slot(slots, i, n_slots, status) : -1;
   uint64_t same = __ballot(sl >= 0);
 #pragma unroll
   for (int bit = 0; bit < 10; ++bit) {           // lanes whose slot agrees with this lane's in every bit
@@ -539,14 +515,14 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
 }
 
 int launch_dispatch(const int32_t* slots, int n, int n_slots, int32_t* hist, int32_t* perm, int32_t* offsets,
-                    int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, hipStream_t st) {
+                    int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, bool zero_status, hipStream_t st) {
   int nchunks = (n + DISPATCH_CHUNK - 1) / DISPATCH_CHUNK;
   if (nchunks == 0) nchunks = 1;
   ProfScope p(st, "prefill_dispatch");
-  dispatch_hist_kernel<<<nchunks, 1024, n_slots * sizeof(int), st>>>(slots, n, n_slots, hist, status);
-  const TileSpec none{0, 1, 0, 1};
+  dispatch_hist_kernel<<<nchunks, 1024, n_slots * sizeof(int), st>>>(slots, n, n_slots, hist, zero_status ? status : nullptr);
+  const TileSpec none{0, 1, 0};
   dispatch_scan_place_kernel<<<nchunks, 1024, n_slots * (sizeof(int) + 16 * sizeof(uint16_t)), st>>>(
-      slots, n, hist, nchunks, n_slots, offsets, spec ? *spec : none, spec ? tiles : nullptr, perm, inv);
+      slots, n, hist, nchunks, n_slots, offsets, spec ? *spec : none, spec ? tiles : nullptr, perm, inv, status);
   return check_launch("prefill dispatch");
 }
 
@@ -560,14 +536,14 @@ int launch_router_logits_small(const RouterSmallArgs& args, hipStream_t st) {
   RouterSmallArgs a = args;
   MIMO_REQUIRE(!a.norm_w || (a.H % 256 == 0 && aligned16(a.norm_w) && a.eps >= 0.0f && a.eps == a.eps),
                MIMO_ERR_ARG, "router: the fused norm needs H a multiple of 256, an aligned weight and eps >= 0");
-  int nquant = (a.xq_hi || (a.norm_w && a.r_out)) ? (int)(((int64_t)a.T * a.H + 255) / 256) : 0;
+  const int nrows = a.norm_w && a.r_out ? (int)((int64_t)a.T * a.H / 256) : 0;
   a.nlog = a.E;
   const int nch = (a.H / 4 + 511) / 512;
   ProfScope p(st, "router_logits_small");
-  switch (nch) {
-    case 2: router_logits_small_kernel<2><<<a.nlog + nquant, 256, 0, st>>>(a); break;
-    default: router_logits_small_kernel<1><<<a.nlog + nquant, 256, 0, st>>>(a); break;
-  }
+  constexpr int RT = 8;
+  const int groups = (a.T + RT - 1) / RT, blocks = a.nlog + (nrows + groups - 1) / groups;
+  if (nch == 2) router_logits_small_kernel<2, RT><<<blocks, 256 * groups, 0, st>>>(a);
+  else router_logits_small_kernel<1, RT><<<blocks, 256 * groups, 0, st>>>(a);
   return check_launch("router_logits_small");
 }
 
@@ -756,7 +732,7 @@ int mimo_prefill_dispatch(const int32_t* slot_inds, int T, int k, int n_slots, i
   MIMO_REQUIRE(ws && ws_bytes >= dispatch_workspace(T * k, n_slots), MIMO_ERR_WORKSPACE,
                "prefill_dispatch: workspace too small");
   return launch_dispatch(slot_inds, T * k, n_slots, static_cast<int32_t*>(ws), perm, offsets, inv, nullptr, nullptr,
-                         nullptr, as_stream(stream));
+                         nullptr, false, as_stream(stream));
 }
 
 }  // extern "C"

@@ -64,7 +64,7 @@ constexpr uint16_t entry(uint32_t bits) {
   return (uint16_t)((v + 0x7FFFu + ((v >> 16) & 1u)) >> 16);
 }
 
-struct Table {
+struct alignas(16) Table {   // 16-byte pieces of it are copied to LDS
   uint16_t v[65536];
 };
 
