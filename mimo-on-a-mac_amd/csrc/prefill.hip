@@ -463,7 +463,7 @@ static PrefillWs carve_prefill(Carve& c, int T, int k, int S, int H, int I, int 
   w.offsets = c.take<int32_t>(S + 1);
   w.tiles = c.take<int4>(1 + (size_t)tl.wcap + tl.scap);
   if (E > 0) {
-    w.logits = c.take<float>((size_t)T * E);
+    w.logits = c.take<float>((size_t)(T <= kRlPartsMax ? kRlParts : 1) * T * E);
     w.inds = c.take<int32_t>(P);
     w.w = c.take<float>(P);
     w.slot_inds = c.take<int32_t>(P);
@@ -621,10 +621,12 @@ static int prefill_block_impl(const uint16_t* x, int T, const uint16_t* Wg, cons
   int32_t* inds = inds_out ? inds_out : pw.inds;
   float* wts = w_out ? w_out : pw.w;
   if (status_out) pw.status = status_out;
-  rc = launch_router_logits(x, Wg, T, bank->hidden, E, pw.logits, st, pw.status);   // clears the status word
+  const bool parts = router_logits_parts(x, Wg, T, bank->hidden);
+  rc = parts ? launch_router_logits_parts(x, Wg, T, bank->hidden, E, pw.logits, st, pw.status)
+             : launch_router_logits(x, Wg, T, bank->hidden, E, pw.logits, st, pw.status);   // clears the status word
   if (rc) return rc;
   rc = launch_router_select(pw.logits, bias, T, E, k, 1.0f, inds, wts, slot_of, pw.slot_inds, bank->n_slots, pw.status,
-                            st);
+                            st, parts);
   if (rc) return rc;
   return run_prefill(x, T, pw.slot_inds, wts, k, bank, nullptr, y, pw, st, false, resid);
 }

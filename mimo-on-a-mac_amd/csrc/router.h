@@ -44,7 +44,13 @@ int launch_router_logits(const uint16_t* x, const uint16_t* W, int T, int H, int
                          int32_t* zero_status = nullptr);
 int launch_router_select(const float* logits, const float* bias, int T, int E, int k, float scaling, int32_t* inds,
                          float* w, const int32_t* slot_of, int32_t* slot_inds, int n_slots, int32_t* status,
-                         hipStream_t st);
+                         hipStream_t st, bool parts = false);
+// Logits of a chunk of at most kRlPartsMax tokens as kRlParts partial sums [kRlParts, T, E], which
+// launch_router_select(parts) adds; router_logits_parts: whether the inputs allow it.
+constexpr int kRlPartsMax = 1024, kRlParts = 8;
+bool router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H);
+int launch_router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H, int E, float* part, hipStream_t st,
+                               int32_t* zero_status);
 // Row tiles of the grouped GEMM: a slot with 1..narrow_max routes is one narrow tile; a larger one is cut into wide
 // tiles of wide_rows routes and one of the remainder.
 // tiles[0] = (wide count, narrow count), wide tile t at tiles[1 + t], narrow tile t at tiles[1 + wcap + t], each

@@ -266,7 +266,11 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const uint16_t* __re
   }
 }
 
-// one wave per row: sigmoid, key, top-k, renormalise; optional expert -> slot mapping for the dispatch
+constexpr int kRlTok = 32, kRlExp = 64, kRlSplit = kRlParts;   // tokens and experts of a prefill logits block, K-ranges
+
+// one wave per row: sigmoid, key, top-k, renormalise; optional expert -> slot mapping for the dispatch.  PARTS > 1: the
+// logits come as PARTS partial sums [PARTS, T, E], added here in that order.
+template <int PARTS>
 __global__ void __launch_bounds__(256) router_select_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                                                             int T, int E, int k, float scaling, int32_t* inds,
                                                             float* w, const int32_t* slot_of, int32_t* slot_inds,
@@ -281,12 +285,19 @@ __global__ void __launch_bounds__(256) router_select_kernel(const float* __restr
   const int t = blockIdx.x * 4 + wave;
   if (t >= T) return;
   if (E <= 256) {   // every logit and bias of the row requested at once, the four sigmoids interleaved
-    float lg[4], bs[4];
+    float lg[4], lp[4][PARTS], bs[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e = lane + 64 * j < E ? lane + 64 * j : 0;
-      lg[j] = logits[(size_t)t * E + e];
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) lp[j][p] = logits[((size_t)p * T + t) * E + e];
       bs[j] = bias[e];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lg[j] = lp[j][0];
+#pragma unroll
+      for (int p = 1; p < PARTS; ++p) lg[j] = lg[j] + lp[j][p];
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -298,7 +309,10 @@ __global__ void __launch_bounds__(256) router_select_kernel(const float* __restr
     }
   } else {
     for (int e = lane; e < E; e += 64) {
-      float s = sigmoid_spec(logits[(size_t)t * E + e]);
+      float l = logits[(size_t)t * E + e];
+#pragma unroll
+      for (int p = 1; p < PARTS; ++p) l = l + logits[((size_t)p * T + t) * E + e];
+      float s = sigmoid_spec(l);
       s_row[e] = s;
       k_row[e] = s + bias[e];
     }
@@ -398,6 +412,7 @@ __global__ void group_routes_kernel(const int32_t* inds, const float* scores, co
 
 // ------------------------------------------------------------------ prefill dispatch (stable counting sort)
 constexpr int DISPATCH_CHUNK = 1024;
+constexpr int kCountChunks = 8;      // up to so many chunks every placement block counts all of them itself
 
 // slot ids outside [0, n_slots) are counted as slot 0 and flagged in *status (never indexed out of bounds)
 __device__ __forceinline__ int checked_slot(const int32_t* slots, int i, int n_slots, int32_t* status) {
@@ -427,33 +442,76 @@ __global__ void __launch_bounds__(1024) dispatch_hist_kernel(const int32_t* __re
 // offsets[s] + sum_{b' < b} hist[b'][s] + (rank among the chunk's routes of slot s).  Block 0 also writes
 // offsets and, with a TileSpec, the row tiles of each slot (see TileSpec).  Ranks within the chunk: earlier
 // waves' counts of the slot (per-wave counts in LDS) plus earlier lanes of the wave (ballots over the slot bits).
+// COUNT: every block counts all chunks itself (no histogram launch before it), and block 0 writes or, when the word
+// holds earlier kernels' flags, lowers the status.
+template <bool COUNT>
 __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t* __restrict__ slots, int n,
                                                                    const int32_t* __restrict__ hist, int nchunks,
                                                                    int n_slots, int32_t* __restrict__ offsets,
                                                                    TileSpec spec, int4* __restrict__ tiles,
                                                                    int32_t* __restrict__ perm, int32_t* __restrict__ inv,
-                                                                   int32_t* status) {
+                                                                   int32_t* status, bool zero_status) {
   extern __shared__ int dsp[];                   // base[n_slots], then wc[16 waves][n_slots] (counts <= 64)
   int* base = dsp;
   uint16_t* wc = reinterpret_cast<uint16_t*>(dsp + n_slots);
   __shared__ int wsum[3][16];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int blk = blockIdx.x;
-  for (int i = tid; i < 16 * n_slots; i += blockDim.x) wc[i] = 0;
-  // per-slot total and the part of it in earlier chunks (integer sums: any order)
-  constexpr int HB = 16;
   int c = 0, pre = 0;
-  if (tid < n_slots)
-    for (int b0 = 0; b0 < nchunks; b0 += HB) {
-      int h[HB];
+  int mine = -1;                                 // COUNT: the thread's route of this chunk
+  if constexpr (COUNT) {
+    // counts in the place of base (all chunks) and of wc (the earlier chunks, n_slots words)
+    int* early = dsp + n_slots;
+    __shared__ int s_bad;
+    int sl[kCountChunks];
 #pragma unroll
-      for (int u = 0; u < HB; ++u) h[u] = b0 + u < nchunks ? hist[(size_t)(b0 + u) * n_slots + tid] : 0;
+    for (int b = 0; b < kCountChunks; ++b) {
+      const int i = b * DISPATCH_CHUNK + tid;
+      sl[b] = b < nchunks && i < n ? slots[i] : -1;
+    }
+    for (int i = tid; i < 2 * n_slots; i += blockDim.x) dsp[i] = 0;
+    if (tid == 0) s_bad = 0;
+    __syncthreads();
 #pragma unroll
-      for (int u = 0; u < HB; ++u) {
-        c += h[u];
-        pre += b0 + u < blk ? h[u] : 0;
+    for (int b = 0; b < kCountChunks; ++b) {
+      const int i = b * DISPATCH_CHUNK + tid;
+      if (b < nchunks && i < n) {
+        int s = sl[b];
+        if (s < 0 || s >= n_slots) {
+          s_bad = 1;
+          s = 0;
+        }
+        atomicAdd(&base[s], 1);                  // integer counts: order independent
+        if (b < blk) atomicAdd(&early[s], 1);
+        if (b == blk) mine = s;
       }
     }
+    __syncthreads();
+    if (tid < n_slots) {
+      c = base[tid];
+      pre = early[tid];
+    }
+    if (status && blk == 0 && tid == 0) {
+      if (zero_status) *status = s_bad ? MIMO_ERR_SLOT : MIMO_OK;
+      else if (s_bad) atomicMin(status, MIMO_ERR_SLOT);
+    }
+    __syncthreads();
+  } else {
+    // per-slot total and the part of it in earlier chunks (integer sums: any order)
+    constexpr int HB = 16;
+    if (tid < n_slots)
+      for (int b0 = 0; b0 < nchunks; b0 += HB) {
+        int h[HB];
+#pragma unroll
+        for (int u = 0; u < HB; ++u) h[u] = b0 + u < nchunks ? hist[(size_t)(b0 + u) * n_slots + tid] : 0;
+#pragma unroll
+        for (int u = 0; u < HB; ++u) {
+          c += h[u];
+          pre += b0 + u < blk ? h[u] : 0;
+        }
+      }
+  }
+  for (int i = tid; i < 16 * n_slots; i += blockDim.x) wc[i] = 0;
   const bool tl = tiles != nullptr && blk == 0;
   const int nw = (tl && c > spec.narrow_max) ? (c + spec.wide_rows - 1) / spec.wide_rows : 0;
   const int ns = (tl && c >= 1 && c <= spec.narrow_max) ? 1 : 0;
@@ -495,7 +553,7 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   }
   // placement of this chunk's routes (slot ids clamped as dispatch_hist_kernel counted them, bad ones flagged)
   const int i = blk * DISPATCH_CHUNK + tid;
-  const int sl = i < n ? checked_slot(slots, i, n_slots, status) : -1;
+  const int sl = COUNT ? mine : (i < n ? checked_slot(slots, i, n_slots, status) : -1);
   uint64_t same = __ballot(sl >= 0);
 #pragma unroll
   for (int bit = 0; bit < 10; ++bit) {           // lanes whose slot agrees with this lane's in every bit
@@ -514,15 +572,25 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   }
 }
 
+// Up to kCountChunks chunks one launch, which counts in every block; more take a histogram launch first (8 blocks
+// counting 8 chunks each cost less than the launch; the counting grows with the square of the chunks).
 int launch_dispatch(const int32_t* slots, int n, int n_slots, int32_t* hist, int32_t* perm, int32_t* offsets,
                     int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, bool zero_status, hipStream_t st) {
   int nchunks = (n + DISPATCH_CHUNK - 1) / DISPATCH_CHUNK;
   if (nchunks == 0) nchunks = 1;
   ProfScope p(st, "prefill_dispatch");
-  dispatch_hist_kernel<<<nchunks, 1024, n_slots * sizeof(int), st>>>(slots, n, n_slots, hist, zero_status ? status : nullptr);
   const TileSpec none{0, 1, 0};
-  dispatch_scan_place_kernel<<<nchunks, 1024, n_slots * (sizeof(int) + 16 * sizeof(uint16_t)), st>>>(
-      slots, n, hist, nchunks, n_slots, offsets, spec ? *spec : none, spec ? tiles : nullptr, perm, inv, status);
+  const size_t lds = n_slots * (sizeof(int) + 16 * sizeof(uint16_t));
+  if (nchunks <= kCountChunks) {
+    dispatch_scan_place_kernel<true><<<nchunks, 1024, lds, st>>>(slots, n, nullptr, nchunks, n_slots, offsets,
+                                                                 spec ? *spec : none, spec ? tiles : nullptr, perm, inv,
+                                                                 status, zero_status);
+    return check_launch("prefill dispatch");
+  }
+  dispatch_hist_kernel<<<nchunks, 1024, n_slots * sizeof(int), st>>>(slots, n, n_slots, hist, zero_status ? status : nullptr);
+  dispatch_scan_place_kernel<false><<<nchunks, 1024, lds, st>>>(slots, n, hist, nchunks, n_slots, offsets,
+                                                                spec ? *spec : none, spec ? tiles : nullptr, perm, inv,
+                                                                status, zero_status);
   return check_launch("prefill dispatch");
 }
 
@@ -554,8 +622,6 @@ int launch_router_logits_small(const RouterSmallArgs& args, hipStream_t st) {
 // of token row i and of expert row i at columns 8g .. 8g + 7 (the same columns for both operands, so the
 // product pairs them correctly whatever order the unit sums in).  The 8 partial tiles are added in LDS in wave
 // order.  Rows past T or E read the last valid row and are not written.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int kRlTok = 32, kRlExp = 64, kRlSplit = 8;
 
 __global__ void __launch_bounds__(512) router_logits_mfma_kernel(const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ W, int T, int H, int E,
@@ -631,6 +697,66 @@ __global__ void __launch_bounds__(512) router_logits_mfma_kernel(const uint16_t*
   }
 }
 
+// The same products for chunks of few tokens, where blocks of 64 experts and the whole reduction are too few: a block
+// (4 waves) takes 32 tokens x 64 experts and one K-range of the 8, a wave 16 of the experts, and the partial sums go to
+// part [8, T, E].  A block's loads bound both kernels: with 24 tokens 4 blocks of 768 KB each took 24.6 us, 32 blocks of
+// 96 KB take 8.7; with 512, 29 and 17.9.  Each partial is summed as router_logits_mfma_kernel sums it and the selection adds them in the same
+// order, so the logits are the same bits.
+__global__ void __launch_bounds__(256) router_logits_parts_kernel(const uint16_t* __restrict__ x,
+                                                                  const uint16_t* __restrict__ W, int T, int H, int E,
+                                                                  float* __restrict__ part, int32_t* zero_status) {
+  if (zero_status && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) *zero_status = 0;
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t0 = blockIdx.y * kRlTok, e0 = blockIdx.x * kRlExp + 16 * wave;
+  const int KW = H / kRlSplit, kb = blockIdx.z * KW;
+  const uint4* xa[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+    xa[a] = reinterpret_cast<const uint4*>(x + (size_t)min(t0 + 16 * a + i, T - 1) * H + kb + 8 * g);
+  const uint4* wb = reinterpret_cast<const uint4*>(W + (size_t)min(e0 + i, E - 1) * H + kb + 8 * g);
+  v4f acc[2] = {v4f{0.0f, 0.0f, 0.0f, 0.0f}, v4f{0.0f, 0.0f, 0.0f, 0.0f}};
+  const int steps = KW / 32;
+  constexpr int U = 8;                               // steps whose loads are in flight at once
+  for (int s0 = 0; s0 < steps; s0 += U) {
+    uint4 av[U][2], bv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = min(s0 + u, steps - 1);
+      av[u][0] = xa[0][4 * s];
+      av[u][1] = xa[1][4 * s];
+      bv[u] = wb[4 * s];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s0 + u < steps)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+          acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[u][a]),
+                                                           __builtin_bit_cast(bf16x8, bv[u]), acc[a], 0, 0, 0);
+  }
+  float* out = part + (size_t)blockIdx.z * T * E;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int t = t0 + 16 * a + 4 * g + q, e = e0 + i;
+      if (t < T && e < E) out[(size_t)t * E + e] = acc[a][q];
+    }
+}
+
+bool router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H) {
+  return T <= kRlPartsMax && H % (kRlSplit * 32) == 0 && aligned16(x) && aligned16(W);
+}
+
+int launch_router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H, int E, float* part, hipStream_t st,
+                               int32_t* zero_status) {
+  ProfScope p(st, "router_logits");
+  dim3 grid((E + kRlExp - 1) / kRlExp, (T + kRlTok - 1) / kRlTok, kRlSplit);
+  router_logits_parts_kernel<<<grid, 256, 0, st>>>(x, W, T, H, E, part, zero_status);
+  return check_launch("router_logits_parts");
+}
+
 int launch_router_logits(const uint16_t* x, const uint16_t* W, int T, int H, int E, float* logits, hipStream_t st,
                          int32_t* zero_status) {
   ProfScope p(st, "router_logits");
@@ -646,11 +772,12 @@ int launch_router_logits(const uint16_t* x, const uint16_t* W, int T, int H, int
 
 int launch_router_select(const float* logits, const float* bias, int T, int E, int k, float scaling, int32_t* inds,
                          float* w, const int32_t* slot_of, int32_t* slot_inds, int n_slots, int32_t* status,
-                         hipStream_t st) {
+                         hipStream_t st, bool parts) {
   int blocks = (T + 3) / 4;
   ProfScope p(st, "router_select");
-  router_select_kernel<<<blocks, 256, 4 * 2 * E * sizeof(float), st>>>(logits, bias, T, E, k, scaling, inds, w,
-                                                                         slot_of, slot_inds, n_slots, status);
+  auto kernel = parts ? router_select_kernel<kRlSplit> : router_select_kernel<1>;
+  kernel<<<blocks, 256, 4 * 2 * E * sizeof(float), st>>>(logits, bias, T, E, k, scaling, inds, w, slot_of, slot_inds,
+                                                         n_slots, status);
   return check_launch("router_select");
 }
 
