@@ -21,7 +21,7 @@ namespace mimo {
 struct PrefillArgs {
   const uint16_t* x;      // [T, H] bf16
   const int32_t* perm;    // sorted position -> flat route
-  const int4* tiles;      // [0] = (wide tiles, narrow tiles); wide at 1 + t, narrow at 1 + wcap + t: (slot, beg, end, 0)
+  const int4* tiles;      // the tile table (TileSpec)
   int wcap, k, H, I;
   // slots [0, S0) address the bank's pools, later ones the staging bank's (pool index 1, slot - S0)
   int S0;
@@ -33,8 +33,7 @@ struct PrefillArgs {
 };
 
 // Row tiles: a slot with at most PF_NARROW_MAX routes is one narrow tile, a larger one is cut into wide tiles of
-// PF_WIDE_ROWS routes and a remainder.  A tile runs the shape of its NJ = ceil(routes / 16) rounded up to 2, 4, 6 or 8
-// chunks of 16 routes.
+// PF_WIDE_ROWS routes and a remainder.  A tile runs the shape of its NJ = ceil(routes / 16) chunks of 16 routes.
 //
 // A K-step is 128 codes.  Per step a wave loads 16 bytes per lane of each of its 4 weight tiles of 16 rows (lane
 // (i, g) = (l % 16, l / 16): codes 32 g .. of row i, which share one E8M0 scale), DEPTH steps ahead of their use, and
@@ -67,9 +66,9 @@ template <bool SMALL> struct PfKind {
 template <int NJ, bool SMALL> struct PfShape : PfKind<SMALL> {
   using Kind = PfKind<SMALL>;
   static constexpr int STAGE = NJ * PF_UNIT * 256;
-  static constexpr int STAGES = NJ >= 6 ? 2 : (NJ == 4 || SMALL ? 3 : 4);
+  static constexpr int STAGES = NJ >= 6 ? 2 : (NJ >= 3 || SMALL ? 3 : 4);
   static constexpr int AHEAD = STAGES - 1;
-  static constexpr int DEPTH = NJ >= 6 ? 2 : (NJ == 4 || SMALL ? 4 : 8);
+  static constexpr int DEPTH = NJ >= 6 ? 2 : (NJ >= 3 || SMALL ? 4 : 8);
   // Weights are requested LU steps at a time, 64 LU consecutive bytes of a row back to back, once the registers of LU
   // steps are free; EARLY steps of them before the first activation rows (whose addresses take a round trip to the
   // route list).
@@ -338,27 +337,34 @@ __device__ __forceinline__ void pf_tile(const PrefillArgs& a, uint8_t* pl, int s
 }
 
 // One launch per GEMM.  Workgroups go to the 8 XCDs round robin (hardware block b runs on XCD b % 8); XCD x takes the
-// x-th eighth of the wide (tile, output block) pairs, then the x-th eighth of the narrow ones, a tile's output blocks
-// one after the other (they share its activations in L2).  The 1-D grid has room for the tile table's capacity; blocks
-// past the used pairs exit at once.
+// x-th share of the wide (tile, output block) pairs, of equal cost (by count, a popular slot's tiles left one XCD up to
+// 13% more work than the average at 2048 tokens), then the x-th eighth of the narrow ones, a tile's output blocks one
+// after the other (they share its activations in L2).  The 1-D grid has room for the tile table's capacity; blocks past
+// the used pairs exit at once.
 template <bool GATEUP, bool SMALL>
 __global__ void __launch_bounds__(256, PfKind<SMALL>::BLOCKS) prefill_gemm_kernel(PrefillArgs a) {
   extern __shared__ __align__(256) uint8_t pl[];
-  const int4 hdr = a.tiles[0];                   // (wide tiles, narrow tiles)
-  const int nw = __builtin_amdgcn_readfirstlane(hdr.x), nn = __builtin_amdgcn_readfirstlane(hdr.y);
-  const int obn = GATEUP ? a.I / (PF_ROWS / 2) : a.H / PF_ROWS;   // output blocks per tile
   const int x = blockIdx.x & 7;
   int j = blockIdx.x >> 3;
-  const int perw = (nw * obn + 7) / 8, pern = (nn * obn + 7) / 8;
-  int at = 1, n = nw * obn, l = x * perw + j;
-  if (j >= perw) {
-    j -= perw;
-    at += a.wcap;
-    n = nn * obn;
-    l = x * pern + j;
-    if (j >= pern) return;
+  const int4 hdr = a.tiles[0], c0 = a.tiles[1 + x], c1 = a.tiles[1 + min(x + 1, 7)];
+  const int nw = __builtin_amdgcn_readfirstlane(hdr.x), nn = __builtin_amdgcn_readfirstlane(hdr.y);
+  const int obn = GATEUP ? a.I / (PF_ROWS / 2) : a.H / PF_ROWS;   // output blocks per tile
+  auto start = [&](int4 c) {                     // first pair of a share
+    return __builtin_amdgcn_readfirstlane(c.x * obn + (c.y * obn + 8 * c.z - 1) / (8 * c.z));
+  };
+  int at = kTileHead, l = 0, n = 0;
+  if (nw > 0) {
+    l = start(c0);
+    n = (x < 7 ? start(c1) : nw * obn) - l;
   }
-  if (l >= n) return;
+  l += j;
+  if (j >= n) {
+    const int per = (nn * obn + 7) / 8;
+    j -= n;
+    at += a.wcap;
+    l = x * per + j;
+    if (j >= per || l >= nn * obn) return;
+  }
   const int tile = l / obn, ob = l - tile * obn;
   const int4 tt = a.tiles[at + tile];
   const int slot = __builtin_amdgcn_readfirstlane(tt.x), beg = __builtin_amdgcn_readfirstlane(tt.y);
@@ -368,8 +374,11 @@ __global__ void __launch_bounds__(256, PfKind<SMALL>::BLOCKS) prefill_gemm_kerne
     else pf_tile<GATEUP, 2, true>(a, pl, slot, beg, nv, ob);
   } else {
     if (nv <= 32) pf_tile<GATEUP, 2, false>(a, pl, slot, beg, nv, ob);
+    else if (nv <= 48) pf_tile<GATEUP, 3, false>(a, pl, slot, beg, nv, ob);
     else if (nv <= 64) pf_tile<GATEUP, 4, false>(a, pl, slot, beg, nv, ob);
+    else if (nv <= 80) pf_tile<GATEUP, 5, false>(a, pl, slot, beg, nv, ob);
     else if (nv <= 96) pf_tile<GATEUP, 6, false>(a, pl, slot, beg, nv, ob);
+    else if (nv <= 112) pf_tile<GATEUP, 7, false>(a, pl, slot, beg, nv, ob);
     else pf_tile<GATEUP, 8, false>(a, pl, slot, beg, nv, ob);
   }
 }
@@ -461,7 +470,7 @@ static PrefillWs carve_prefill(Carve& c, int T, int k, int S, int H, int I, int 
   w.perm = c.take<int32_t>(P);
   w.inv = c.take<int32_t>(P);
   w.offsets = c.take<int32_t>(S + 1);
-  w.tiles = c.take<int4>(1 + (size_t)tl.wcap + tl.scap);
+  w.tiles = c.take<int4>(kTileHead + (size_t)tl.wcap + tl.scap);
   if (E > 0) {
     w.logits = c.take<float>((size_t)(T <= kRlPartsMax ? kRlParts : 1) * T * E);
     w.inds = c.take<int32_t>(P);
@@ -516,9 +525,12 @@ static int run_prefill(const uint16_t* x, int T, const int32_t* slot_inds, const
   if (!rc) rc = pf_allow_lds<false, false>();
   if (rc) return rc;
   // 1-D grids with an index on every XCD for each of its (tile, output block) pairs of either kind; blocks past the
-  // used pairs exit at once
+  // used pairs exit at once.  A wide tile costs at least kTileCost + 1, all of them at most `cost`, and a share holds an
+  // eighth of the cost and less than one tile more.
+  const int64_t cost = (int64_t)(kTileCost + 1) * tl.wcap + P / PF_UNIT;
   auto grid_of = [&](int obn) {
-    return 8 * (int)(((int64_t)tl.wcap * obn + 7) / 8 + ((int64_t)tl.scap * obn + 7) / 8);
+    const int64_t wide = (cost / 8 + 1 + kTileCost + tl.rows / PF_UNIT) * obn / (kTileCost + 1) + 2;
+    return 8 * (int)(wide + ((int64_t)tl.scap * obn + 7) / 8);
   };
   { ProfScope p(st, "prefill_gateup");
     const int grid = grid_of(I / (PF_ROWS / 2));

@@ -47,14 +47,17 @@ int launch_router_select(const float* logits, const float* bias, int T, int E, i
                          hipStream_t st, bool parts = false);
 // Logits of a chunk of at most kRlPartsMax tokens as kRlParts partial sums [kRlParts, T, E], which
 // launch_router_select(parts) adds; router_logits_parts: whether the inputs allow it.
-constexpr int kRlPartsMax = 1024, kRlParts = 8;
+constexpr int kRlPartsMax = 640, kRlParts = 8;
 bool router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H);
 int launch_router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H, int E, float* part, hipStream_t st,
                                int32_t* zero_status);
 // Row tiles of the grouped GEMM: a slot with 1..narrow_max routes is one narrow tile; a larger one is cut into wide
 // tiles of wide_rows routes and one of the remainder.
-// tiles[0] = (wide count, narrow count), wide tile t at tiles[1 + t], narrow tile t at tiles[1 + wcap + t], each
-// (slot, first route, end route, 0).
+// tiles[0] = (wide count, narrow count, 0, 0), wide tile t at tiles[kTileHead + t], narrow tile t at
+// tiles[kTileHead + wcap + t], each (slot, first route, end route, 0).  tiles[1 + x] cuts the wide tiles into eight
+// shares of equal cost, a tile costing kTileCost plus its chunks of 16 routes: share x starts off / (8 cost) of the way
+// through tile t, for (t, off, cost, 0) (not written without wide tiles).
+constexpr int kTileHead = 9, kTileCost = 2;
 struct TileSpec {
   int narrow_max, wide_rows, wcap;
 };

@@ -414,7 +414,7 @@ __global__ void group_routes_kernel(const int32_t* inds, const float* scores, co
 
 // ------------------------------------------------------------------ prefill dispatch (stable counting sort)
 constexpr int DISPATCH_CHUNK = 1024;
-constexpr int kCountChunks = 8;      // up to so many chunks every placement block counts all of them itself
+constexpr int kCountChunks = 16;      // up to so many chunks every placement block counts all of them itself
 
 // slot ids outside [0, n_slots) are counted as slot 0 and flagged in *status (never indexed out of bounds)
 __device__ __forceinline__ int checked_slot(const int32_t* slots, int i, int n_slots, int32_t* status) {
@@ -456,7 +456,7 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   extern __shared__ int dsp[];                   // base[n_slots], then wc[16 waves][n_slots] (counts <= 64)
   int* base = dsp;
   uint16_t* wc = reinterpret_cast<uint16_t*>(dsp + n_slots);
-  __shared__ int wsum[3][16];
+  __shared__ int wsum[4][16];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int blk = blockIdx.x;
   int c = 0, pre = 0;
@@ -517,25 +517,32 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   const bool tl = tiles != nullptr && blk == 0;
   const int nw = (tl && c > spec.narrow_max) ? (c + spec.wide_rows - 1) / spec.wide_rows : 0;
   const int ns = (tl && c >= 1 && c <= spec.narrow_max) ? 1 : 0;
-  int v0 = c, v1 = nw, v2 = ns;                  // inclusive scans within the wave
+  const int full = spec.wide_rows / 16 + kTileCost;    // cost of a full wide tile
+  const int last = nw ? (c - spec.wide_rows * (nw - 1) + 15) / 16 + kTileCost : 0;
+  const int cost = nw ? full * (nw - 1) + last : 0;
+  int v0 = c, v1 = nw, v2 = ns, v3 = cost;       // inclusive scans within the wave
   for (int d = 1; d < 64; d <<= 1) {
     const int u0 = __shfl_up(v0, d, 64), u1 = __shfl_up(v1, d, 64), u2 = __shfl_up(v2, d, 64);
+    const int u3 = __shfl_up(v3, d, 64);
     if (lane >= d) {
       v0 += u0;
       v1 += u1;
       v2 += u2;
+      v3 += u3;
     }
   }
   if (lane == 63) {
     wsum[0][wv] = v0;
     wsum[1][wv] = v1;
     wsum[2][wv] = v2;
+    wsum[3][wv] = v3;
   }
   __syncthreads();
   for (int w = 0; w < wv; ++w) {
     v0 += wsum[0][w];
     v1 += wsum[1][w];
     v2 += wsum[2][w];
+    v3 += wsum[3][w];
   }
   if (tid < n_slots) {
     const int e0 = v0 - c, e1 = v1 - nw, e2 = v2 - ns;   // exclusive prefixes
@@ -547,10 +554,17 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
         if (tiles) tiles[0] = make_int4(v1, v2, 0, 0);
       }
       if (nw) {
-        for (int q = 0; q < nw; ++q)
-          tiles[1 + e1 + q] = make_int4(tid, e0 + spec.wide_rows * q, e0 + min(spec.wide_rows * (q + 1), c), 0);
+        int total = 0;
+        for (int w = 0; w < 16; ++w) total += wsum[3][w];
+        for (int q = 0; q < nw; ++q) {
+          tiles[kTileHead + e1 + q] = make_int4(tid, e0 + spec.wide_rows * q, e0 + min(spec.wide_rows * (q + 1), c), 0);
+          // the shares that start within this tile: 8 cum <= total x < 8 (cum + cost)
+          const int cum = v3 - cost + full * q, tc = q == nw - 1 ? last : full;
+          for (int x = (int)((8ll * cum + total - 1) / total); x < 8 && (int64_t)total * x < 8ll * (cum + tc); ++x)
+            tiles[1 + x] = make_int4(e1 + q, (int)((int64_t)total * x - 8ll * cum), tc, 0);
+        }
       }
-      if (ns) tiles[1 + spec.wcap + e2] = make_int4(tid, e0, e0 + c, 0);
+      if (ns) tiles[kTileHead + spec.wcap + e2] = make_int4(tid, e0, e0 + c, 0);
     }
   }
   // placement of this chunk's routes (slot ids clamped as dispatch_hist_kernel counted them, bad ones flagged)

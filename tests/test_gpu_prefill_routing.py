@@ -1,5 +1,5 @@
-"""The prefill chunk's routing launches at the sizes where their shape changes: logits as partial sums (up to 1024
-tokens) or whole, the dispatch counting in its own blocks (up to 8192 routes) or after a histogram launch."""
+"""The prefill chunk's routing launches at the sizes where their shape changes: logits as partial sums (up to 640
+tokens) or whole, the dispatch counting in its own blocks (up to 16384 routes) or after a histogram launch."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +10,7 @@ from helpers import rand_bf16, to_dev_bf16, zipf_routes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T", [9, 31, 33, 1023, 1024, 1025])
+@pytest.mark.parametrize("T", [9, 31, 33, 639, 640, 641])
 @pytest.mark.parametrize("H,E,k", [(256, 8, 2), (768, 70, 3), (1024, 300, 5)])
 def test_block_routes_are_the_routers(rng, T, H, E, k):
     """The block's routes and weights equal the router entry point's (whole logits) bit for bit."""
@@ -29,7 +29,8 @@ def test_block_routes_are_the_routers(rng, T, H, E, k):
 
 
 @pytest.mark.parametrize("T,k,S", [(1, 1, 1), (128, 8, 256), (129, 8, 256), (1023, 8, 1024), (1024, 8, 256),
-                                   (1025, 8, 256), (2049, 4, 7)])
+                                   (1025, 8, 256), (2049, 4, 7),
+                                   (2048, 8, 256), (2049, 8, 256)])
 def test_dispatch_against_oracle(rng, T, k, S):
     from mimo_stream import prefill_dispatch
     inds = zipf_routes(rng, T, max(S, k), k) % S
