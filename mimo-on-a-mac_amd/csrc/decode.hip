@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
     const uint16_t gt = f32_to_bf16(gsum);
     const float gtf = bf16_to_f32(gt);
     const float ut = round_bf16(usum);
-    const float sig = round_bf16(sigmoid_spec(gtf));   // the bf16 sigmoid table's entry for gt, computed in place
+    const float sig = sigmoid_bf16(gtf);               // the bf16 sigmoid table's entry for gt, computed in place
     const uint16_t hb = f32_to_bf16(round_bf16(gtf * sig) * ut);
     if (e_r < cnt || (a.zero_pad && e_r < a.R))   // padding rows (zeros) only for callers that asked for h
       a.h[((size_t)u * a.R + e_r) * a.I + n0 + e_n] = e_r < cnt ? hb : (uint16_t)0;

@@ -113,6 +113,24 @@ __device__ __forceinline__ float sigmoid_spec(float xf) {
   return nan ? __uint_as_float(0x7FC00000u) : s;
 }
 
+// round_bf16(sigmoid_spec(x)) for a bf16 x, through the hardware exponential and reciprocal: their fp32 result is within
+// 8 units of its last place (x log2 e split so that its fraction is exact to the last bits; 1 ulp each from v_exp_f32,
+// the addition and v_rcp_f32), so it rounds to the same bf16 unless it lies that close to the middle between two; those,
+// and arguments past 80, take the specified evaluation (some 1,000 cycles of dependent fp64).
+__device__ __forceinline__ float sigmoid_bf16(float x) {
+#pragma clang fp contract(off)
+  constexpr float kHi = 0x1.714p+0f, kLo = 0x1.47652b8p-12f;   // log2 e: 13 bits (times 8 of x: exact), the rest
+  const float t = -x * kHi;
+  const float n = __builtin_rintf(t);
+  const float f = (t - n) - x * kLo;
+  const float e = __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+  const float s = __builtin_amdgcn_rcpf(1.0f + e);
+  const int off = (int)(__float_as_uint(s) & 0xFFFFu) - 0x8000;
+  const bool sure = fabsf(x) <= 80.0f && (off > 32 || off < -32);
+  if (sure) return round_bf16(s);
+  return round_bf16(sigmoid_spec(x));
+}
+
 // 32 bf16-valued floats -> hi / lo E4M3 words (4 codes per word, element order) and E8M0 bytes: hi = E4M3 block
 // quantisation of v, lo = the same of the exact residual v - hi.  Codes from the hardware conversion
 // (v_cvt_pk_fp8_f32: OCP E4M3, round to nearest even, checked against the oracle on every bf16 input;
