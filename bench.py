@@ -41,8 +41,7 @@ ROUTER_BYTES = E * H * 2
 GATEUP_BYTES_PER_EXPERT = 2 * (I * H // 2 + I * H // 32)      # 8,912,896
 FLOPS_PER_ROUTE = 2 * (2 * I * H + H * I)                      # 50,331,648
 PF_HOT_EXPERTS = 16          # concentrated prefill: every token's 8 experts among 16 (1,024 routes each at 2048)
-HILO_CEILING_TFLOPS = 2500.0  # useful flops when each product takes two fp8 x fp4 MFMAs at the 5.0 PF fp8 peak
-ISSUE_RATE_TFLOPS = 3310.0    # issued fp8 x fp4 MFMA flops at the rate a throughput probe measured (48.6 cycles)
+BF16_PEAK_TFLOPS = 2500.0    # dense bf16 MFMA peak: the expert products run on v_mfma_f32_16x16x32_bf16
 
 
 def log(*a):
@@ -286,10 +285,9 @@ def prefill_case(layers, T, steps, warmup, seed, device, timed=True, routes=None
 
 
 def hot_prefill_case(layers, T, device):
-    """Prefill with every route on PF_HOT_EXPERTS experts (hot_routes): only full wide tiles of popular experts,
-    the GEMMs' compute-bound case.  Per GEMM: useful TFLOP/s (one product = 2 flops per multiply-add), against
-    the hi/lo ceiling (2 fp8 x fp4 MFMAs per product at the 5.0 PF fp8 peak) and, as issued MFMA flops (hi + lo),
-    against the issue rate a throughput probe of the same instruction measured."""
+    """Prefill with every route on PF_HOT_EXPERTS experts (hot_routes): only full tiles of popular experts, the GEMMs'
+    compute-bound case.  Per GEMM: useful TFLOP/s (one product = 2 flops per multiply-add), against the dense bf16
+    MFMA peak and the MXFP4 one."""
     r = prefill_case(layers, T, 20, 3, seed=0, device=device, routes=hot_routes(T, 60 + T, 4))
     kt = kernel_times(r.pop("_fn"), 4)
     r["kernel_us"] = {k: round(v[0] * 1e3, 1) for k, v in kt.items()}
@@ -299,8 +297,7 @@ def hot_prefill_case(layers, T, device):
                              ("down", "prefill_down", T * K * 2 * (H * I))):
         us = kt[kern][0] * 1e3
         useful = flops / (us * 1e-6) / 1e12
-        r[tag] = {"us": round(us, 1), "useful_TFLOPs": useful, "hilo_ceiling_frac": useful / HILO_CEILING_TFLOPS,
-                  "issued_vs_probe_rate": 2 * useful / ISSUE_RATE_TFLOPS,
+        r[tag] = {"us": round(us, 1), "useful_TFLOPs": useful, "bf16_mfma_frac": useful / BF16_PEAK_TFLOPS,
                   "mxfp4_mfma_frac": useful / MXFP4_PEAK_TFLOPS}
     return r
 
@@ -341,7 +338,12 @@ def stack_case(layers, M, tokens, device, seed, popularity="zipf"):
             "hbm_frac": nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
 
 
-HEADLINE_KERNEL = ("decode_gateup_kernel<8, true, false, true>", 32768, 8)   # 1-row decode: 128 x 8 blocks of 256
+HEADLINE_GRID = (32768, 8)   # 1-row decode: 128 x 8 blocks of 256
+
+
+def is_headline(key):
+    """Whether a trace's (kernel, grid x, grid y, ...) is the 1-row gate/up launch (any further template arguments)."""
+    return key[0].startswith("decode_gateup_kernel<8, true, false") and tuple(key[1:3]) == HEADLINE_GRID
 
 
 def trace_parse(d, out_path=None):
@@ -367,19 +369,19 @@ def trace_parse(d, out_path=None):
             key = (n.split("(")[0].replace("void ", "").replace("mimo::", ""), int(r["Grid_Size_X"]),
                    int(r["Grid_Size_Y"]), int(r["Workgroup_Size_X"]))
             acc[key].append((t1 - t0) / 1e3)
-            if key[:3] == HEADLINE_KERNEL and q in prev_end:
+            if is_headline(key) and q in prev_end:
                 gap.append((t1 - prev_end[q]) / 1e3)
         prev_end[q] = t1
     print("| kernel | grid (threads) | block | dispatches | avg µs | min µs | max µs |\n|---|---|---|---|---|---|---|")
     for (n, gx, gy, wx), v in sorted(acc.items()):
         print(f"| `{n}` | {gx}×{gy} | {wx} | {len(v)} | {sum(v) / len(v):.2f} | {min(v):.2f} | {max(v):.2f} |")
-    head = [v for k, v in acc.items() if k[:3] == HEADLINE_KERNEL]
+    head = [(k, v) for k, v in acc.items() if is_headline(k)]
     if head:
-        v = head[0]
+        k, v = head[0]
         out = {"decode_gateup_kernel:decode_m1": {
             "avg_us": sum(v) / len(v), "launches": len(v),
             "after_previous_end_us": sum(gap) / len(gap) if gap else None}}
-        print(f"\nHeadline kernel `{HEADLINE_KERNEL[0]}` (grid {HEADLINE_KERNEL[1]}×{HEADLINE_KERNEL[2]}): "
+        print(f"\nHeadline kernel `{k[0]}` (grid {k[1]}×{k[2]}): "
               f"{len(v)} dispatches, average duration {out['decode_gateup_kernel:decode_m1']['avg_us']:.2f} µs; "
               f"average interval from the previous kernel's end on its queue to its own end "
               f"{out['decode_gateup_kernel:decode_m1']['after_previous_end_us']:.2f} µs (the interval the "
@@ -512,20 +514,9 @@ def _counter_rows(d):
     return rows
 
 
-def gemm_kernels(gate):
-    """Kernel-name tests for the two launches of one prefill GEMM: (narrow tiles, wide tiles)."""
-    g = "true" if gate else "false"
-    return (lambda n: f"prefill_gemm_kernel<{g}, false>" in n), (lambda n: f"prefill_gemm_kernel<{g}, true>" in n)
-
-
-def per_layer(vals_narrow, vals_wide, combine=lambda a, b: a + b):
-    """One value per prefill layer from the per-dispatch values of its narrow and wide launches (dispatch
-    order; a layer without narrow tiles has no narrow launch only when no layer has one)."""
-    if not vals_narrow:
-        return list(vals_wide)
-    if len(vals_narrow) != len(vals_wide):
-        raise SystemExit(f"{len(vals_narrow)} narrow vs {len(vals_wide)} wide launches")
-    return [combine(a, b) for a, b in zip(vals_narrow, vals_wide)]
+def gemm_kernel(gate):
+    """Kernel-name test for the launch of one prefill GEMM (either of its two configurations)."""
+    return lambda n: f"prefill_gemm_kernel<{'true' if gate else 'false'}," in n
 
 
 def traffic_parse(fetch_dir, write_dir):
@@ -562,24 +553,18 @@ def traffic_parse(fetch_dir, write_dir):
                        "algorithmic_bytes": algo, "fetch_scale": fetch_scale, "write_scale": write_scale,
                        "calibration": "elementwise multiply by one over 1 GiB: reads and writes 1 GiB"}}
     rows = [("decode_gateup_kernel (1 row, 8 experts)", len(gf), fetch, write, algo)]
-    # prefill GEMMs of the payload: algorithmic bytes = distinct experts' weights and scales + activation codes
-    # and scales read + results written (hi/lo E4M3 h with scales, or bf16 Y)
+    # prefill GEMMs of the payload: algorithmic bytes = distinct experts' weights and scales + activation rows
+    # read + results written (bf16 h or Y)
     import numpy as np
     T, P = PF_TRAFFIC_T, PF_TRAFFIC_T * K
     routes = zipf_routes(T, 20 + T, 4)
     U = float(np.mean([len(np.unique(routes[s % 4][0])) for s in range(PF_TRAFFIC_STEPS)]))
-    split = lambda rows_, cols: 2 * rows_ * cols + 2 * rows_ * cols // 32          # hi + lo codes and scales
-    algo_pf = {True: U * GATEUP_BYTES_PER_EXPERT + split(T, H) + split(P, I),
-               False: U * (H * I // 2 + H * I // 32) + split(P, I) + P * H * 2}
-    def layer_vals(acc, gate):
-        kn, kw = gemm_kernels(gate)
-        vn = [v for n in acc if kn(n) for v in acc[n]]
-        _, vw = pick(acc, kw)
-        return per_layer(vn, vw)
+    algo_pf = {True: U * GATEUP_BYTES_PER_EXPERT + 2 * T * H + 2 * P * I,
+               False: U * (H * I // 2 + H * I // 32) + 2 * P * I + 2 * P * H}
     for gate in (True, False):
-        pname = f"prefill_gemm_kernel<{'true' if gate else 'false'}, narrow + wide>"
-        pf_ = layer_vals(f, gate)[:PF_TRAFFIC_STEPS]                  # the Zipf layers come first
-        pw_ = layer_vals(w, gate)[:PF_TRAFFIC_STEPS]
+        pname, pf_ = pick(f, gemm_kernel(gate))
+        _, pw_ = pick(w, gemm_kernel(gate))
+        pf_, pw_ = pf_[:PF_TRAFFIC_STEPS], pw_[:PF_TRAFFIC_STEPS]     # the Zipf layers come first
         pfetch = sum(pf_) / len(pf_) * fetch_scale
         pwrite = sum(pw_) / len(pw_) * write_scale
         tag = "prefill_gateup" if gate else "prefill_down"
@@ -587,7 +572,7 @@ def traffic_parse(fetch_dir, write_dir):
         out[f"_detail_{tag}"] = {"kernel": pname, "dispatches": len(pf_), "fetch_bytes": pfetch,
                                  "write_bytes": pwrite, "algorithmic_bytes": algo_pf[gate],
                                  "distinct_experts": U}
-        rows.append((f"prefill {'gate/up' if gate else 'down'} GEMM, narrow + wide launches ({T} tokens, {U:.1f} experts)",
+        rows.append((f"prefill {'gate/up' if gate else 'down'} GEMM ({T} tokens, {U:.1f} experts)",
                      len(pf_), pfetch, pwrite, algo_pf[gate]))
     with open(os.path.join(ROOT, "profiles", "traffic.json"), "w") as fh:
         json.dump(out, fh, indent=1)
@@ -603,9 +588,7 @@ def traffic_parse(fetch_dir, write_dir):
 def mfma_parse(pmc_dir, trace_dir):
     """MFMA work of the prefill GEMMs from a --pmc run (SQ_INSTS_MFMA, SQ_VALU_MFMA_BUSY_CYCLES,
     GRBM_GUI_ACTIVE) and their durations from a --kernel-trace run of the same payload: the Zipf(1.1) layers
-    (the first PF_TRAFFIC_STEPS of each GEMM) and the layers on PF_HOT_EXPERTS experts (the next PF_HOT_STEPS).
-    A GEMM is two concurrent launches (narrow and wide tiles): instructions are summed, its time runs from the
-    first start to the last end of the pair in the trace run."""
+    (the first PF_TRAFFIC_STEPS of each GEMM) and the layers on PF_HOT_EXPERTS experts (the next PF_HOT_STEPS)."""
     import csv
     import glob
     cnt = {}
@@ -622,15 +605,13 @@ def mfma_parse(pmc_dir, trace_dir):
         spans.setdefault(r["Kernel_Name"], []).append((int(r["Start_Timestamp"]), int(r["End_Timestamp"])))
     groups = ((f"2048 tokens, Zipf(1.1)", 0, PF_TRAFFIC_STEPS),
               (f"2048 tokens on {PF_HOT_EXPERTS} experts", PF_TRAFFIC_STEPS, PF_TRAFFIC_STEPS + PF_HOT_STEPS))
-    print("| GEMM | routes | layers | MFMA instr / layer | avg µs | MFMA TFLOP/s issued (hi + lo) | "
-          "useful TFLOP/s | issued / probe rate | useful / hi-lo ceiling | busy cycles / instr |")
-    print("|---|---|---|---|---|---|---|---|---|---|")
+    print("| GEMM | routes | layers | MFMA instr / layer | avg µs | MFMA TFLOP/s issued | "
+          "issued / bf16 peak | busy cycles / instr |")
+    print("|---|---|---|---|---|---|---|---|")
     for gate in (True, False):
-        kn, kw = gemm_kernels(gate)
-        sel = lambda src, key, c=None: [v for n in src if key(n) for v in (src[n][c] if c else src[n])]
-        inst = per_layer(sel(cnt, kn, "SQ_INSTS_MFMA"), sel(cnt, kw, "SQ_INSTS_MFMA"))
-        busy = per_layer(sel(cnt, kn, "SQ_VALU_MFMA_BUSY_CYCLES"), sel(cnt, kw, "SQ_VALU_MFMA_BUSY_CYCLES"))
-        span = per_layer(sel(spans, kn), sel(spans, kw), lambda a, b: (min(a[0], b[0]), max(a[1], b[1])))
+        key = gemm_kernel(gate)
+        sel = lambda src, c=None: [v for n in src if key(n) for v in (src[n][c] if c else src[n])]
+        inst, busy, span = sel(cnt, "SQ_INSTS_MFMA"), sel(cnt, "SQ_VALU_MFMA_BUSY_CYCLES"), sel(spans)
         for label, a, b in groups:
             n = len(inst[a:b])
             if not n or not span[a:b]:
@@ -638,15 +619,13 @@ def mfma_parse(pmc_dir, trace_dir):
             ins = sum(inst[a:b]) / n
             bz = sum(busy[a:b]) / n
             d = sum((e - st) * 1e-9 for st, e in span[a:b]) / len(span[a:b])
-            issued = ins * 16 * 16 * 128 * 2 / d / 1e12
+            issued = ins * 16 * 16 * 32 * 2 / d / 1e12
             print(f"| {'gate/up' if gate else 'down'} | {label} | {n} | {ins:,.0f} | {d * 1e6:.1f} | {issued:.0f} | "
-                  f"{issued / 2:.0f} | {issued / ISSUE_RATE_TFLOPS:.2f} | {issued / 2 / HILO_CEILING_TFLOPS:.2f} | "
-                  f"{bz / ins:.1f} |")
+                  f"{issued / BF16_PEAK_TFLOPS:.2f} | {bz / ins:.1f} |")
 
 
 def pipe_parse(lds_dir, wait_dir):
-    """Where the prefill GEMMs' waves spend their cycles, per launch (narrow or wide tiles; counter runs serialise
-    the two launches of a GEMM) and routing group (as mfma_parse):
+    """Where the prefill GEMMs' waves spend their cycles, per launch and routing group (as mfma_parse):
     LDS utilisation (SQ_LDS_IDX_ACTIVE over GRBM_GUI_ACTIVE of one XCD x 256 CUs), bank conflicts per access,
     MFMA pipe busy per SIMD, and the fractions of wave-cycles waiting (SQ_WAIT_ANY: s_waitcnt and barriers;
     SQ_WAIT_INST_ANY: an instruction waiting to issue) or issuing (SQ_ACTIVE_INST_ANY / _LDS)."""
@@ -669,7 +648,7 @@ def pipe_parse(lds_dir, wait_dir):
             ia, bc = m("SQ_LDS_IDX_ACTIVE", lds), m("SQ_LDS_BANK_CONFLICT", lds)
             g2 = m("GRBM_GUI_ACTIVE", wt) / 8
             wc = m("SQ_WAVE_CYCLES", wt)
-            if ia <= bc or wc <= 0:                      # a launch with no tiles of its shape in these layers
+            if ia <= bc or wc <= 0:
                 continue
             print(f"| {k.split('(')[0].replace('void mimo::', '')} | {label} | {ia / (grbm * 256):.2f} | {bc / (ia - bc):.2f} | "
                   f"{m('SQ_VALU_MFMA_BUSY_CYCLES', wt) / (g2 * 1024):.2f} | {m('SQ_WAIT_ANY', wt) / wc:.2f} | "
