@@ -8,6 +8,12 @@
 // (4 waves, two blocks per CU) owns one row tile and 256 weight rows, 64 per wave.  Weights go from HBM straight to
 // the registers of the one wave that uses them and are turned into bf16 there (exactly: an E2M1 value times a power
 // of two); the bf16 activation rows, which all four waves use, go through an LDS ring.
+//
+// What bounds it: up to ~700 tokens HBM (512 tokens: gate/up and down read 3.4 GB in ~690 us, 5 TB/s; the loads alone
+// take 405 of gate/up's 460 us); above, the MFMAs at the ~1.9 GHz that the chip's power leaves (60% busy at 6250
+// tokens) and the copies that they hide only in part (gate/up 1516 us; without activation copies 1327, without weight
+// loads 1296, without both 1184).  A layer step took 369 / 779 / 1246 / 2807 us at 24 / 512 / 2048 / 6250 tokens with
+// two E4M3 planes per activation on the block-scaled MFMA and two launches per GEMM, and takes 301 / 716 / 1081 / 2392.
 #include <algorithm>
 #include <atomic>
 
@@ -33,7 +39,7 @@ struct PrefillArgs {
 };
 
 // Row tiles: a slot with at most PF_NARROW_MAX routes is one narrow tile, a larger one is cut into wide tiles of
-// PF_WIDE_ROWS routes and a remainder.  A tile runs the shape of its NJ = ceil(routes / 16) chunks of 16 routes.
+// PF_WIDE_ROWS (PF_SMALL_ROWS) routes and a remainder.  A tile runs the shape of its NJ = ceil(routes / 16) chunks of 16 routes.
 //
 // A K-step is 128 codes.  Per step a wave loads 16 bytes per lane of each of its 4 weight tiles of 16 rows (lane
 // (i, g) = (l % 16, l / 16): codes 32 g .. of row i, which share one E8M0 scale), DEPTH steps ahead of their use, and
@@ -45,7 +51,13 @@ struct PrefillArgs {
 // reads are then free of bank conflicts (with the chunk 4 g + m at (4 g + m) ^ (r & 15) they took twice the cycles).
 constexpr int PF_NARROW_MAX = 32;
 constexpr int PF_WIDE_ROWS = 128;
-constexpr int PF_SMALL_AVG = 18;
+// Routes per slot up to which the streaming configuration runs (three blocks per CU, tiles of up to 64 routes), against
+// the other: Zipf routes at 512 tokens (16 a slot) 720 us a layer against 750, 640 (20) 773 against 808, 768 (24) 810
+// against 835, 1024 (32) 906 against 918; near-uniform ones at 700 tokens 779 against 792, at 1000 (31) 872 against 864.
+// Its tiles are not smaller: at 32 routes a popular slot's weights were read and converted twice as often (Zipf, 512
+// tokens: 763 us, 733 with 48).
+constexpr int PF_SMALL_AVG = 24;
+constexpr int PF_SMALL_ROWS = 64;
 constexpr int PF_UNIT = 16;                          // routes per MFMA chunk
 constexpr int PF_ROWS = 256;                         // weight rows per block
 // the part of the bf16 sigmoid table that is not constant: |x| in [2^-9, 128) (below, 0.5; above, 0 or 1)
@@ -58,7 +70,7 @@ constexpr int PF_SC = PF_ROWS * 4 * PF_SCW;          // bytes of one window of t
 // follow it).
 template <bool SMALL> struct PfKind {
   static constexpr int BLOCKS = SMALL ? 3 : 2;
-  static constexpr int RING = SMALL ? 24576 : 65536;
+  static constexpr int RING = SMALL ? 32768 : 65536;
   static constexpr int LDS = RING + 2 * PF_SC;
   static_assert(BLOCKS * LDS <= 163840, "blocks per CU within 160 KB of LDS");
 };
@@ -66,13 +78,13 @@ template <bool SMALL> struct PfKind {
 template <int NJ, bool SMALL> struct PfShape : PfKind<SMALL> {
   using Kind = PfKind<SMALL>;
   static constexpr int STAGE = NJ * PF_UNIT * 256;
-  static constexpr int STAGES = NJ >= 6 ? 2 : (NJ >= 3 || SMALL ? 3 : 4);
+  static constexpr int STAGES = NJ >= 6 || (NJ >= 3 && SMALL) ? 2 : (NJ >= 3 || SMALL ? 3 : 4);
   static constexpr int AHEAD = STAGES - 1;
-  static constexpr int DEPTH = NJ >= 6 ? 2 : (NJ >= 3 || SMALL ? 4 : 8);
+  static constexpr int DEPTH = NJ >= 6 || (NJ >= 3 && SMALL) ? 2 : (NJ >= 3 || SMALL ? 4 : 8);
   // Weights are requested LU steps at a time, 64 LU consecutive bytes of a row back to back, once the registers of LU
   // steps are free; EARLY steps of them before the first activation rows (whose addresses take a round trip to the
   // route list).
-  static constexpr int LU = NJ >= 6 ? 1 : 2;
+  static constexpr int LU = NJ >= 6 || (NJ >= 3 && SMALL) ? 1 : 2;
   static constexpr int EARLY = LU;
   // weight loads issued in the AHEAD steps before step u of a round of DEPTH
   static constexpr int newer(int u) {
@@ -371,7 +383,9 @@ __global__ void __launch_bounds__(256, PfKind<SMALL>::BLOCKS) prefill_gemm_kerne
   const int nv = __builtin_amdgcn_readfirstlane(tt.z - tt.y);
   if constexpr (SMALL) {
     if (nv <= 16) pf_tile<GATEUP, 1, true>(a, pl, slot, beg, nv, ob);
-    else pf_tile<GATEUP, 2, true>(a, pl, slot, beg, nv, ob);
+    else if (nv <= 32) pf_tile<GATEUP, 2, true>(a, pl, slot, beg, nv, ob);
+    else if (nv <= 48) pf_tile<GATEUP, 3, true>(a, pl, slot, beg, nv, ob);
+    else pf_tile<GATEUP, 4, true>(a, pl, slot, beg, nv, ob);
   } else {
     if (nv <= 32) pf_tile<GATEUP, 2, false>(a, pl, slot, beg, nv, ob);
     else if (nv <= 48) pf_tile<GATEUP, 3, false>(a, pl, slot, beg, nv, ob);
@@ -455,7 +469,7 @@ struct PfTiling {
 static PfTiling pf_tiling(int64_t P, int S) {
   PfTiling t;
   t.small = P <= (int64_t)PF_SMALL_AVG * S;
-  t.rows = t.small ? 32 : PF_WIDE_ROWS;
+  t.rows = t.small ? PF_SMALL_ROWS : PF_WIDE_ROWS;
   t.wcap = (int)(P / t.rows + std::min<int64_t>(S, P / (PF_NARROW_MAX + 1)) + 1);
   t.scap = (int)std::min<int64_t>(S, P);
   return t;
