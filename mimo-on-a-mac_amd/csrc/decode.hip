@@ -380,7 +380,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
 // dot products of each route land in LDS (one row per route: expert u's rows start at the sum of the
 // earlier experts' counts); the block adds them in a fixed order, applies the router weight (and the bf16
 // rounding of the gather_qmm path when asked, model.py:181), sums each row's k routes in route order
-// (kernels.py:198-199) and writes y.  No other block is waited for.
+// (kernels.py:198-199) and writes y.  No other block is waited for.  HBM and the round trips before its first weights
+// bound it: 1 row (36 MB) 10.5 us, 11.0 with h as two E4M3 planes split here.
 
 // Per-wave LDS buffer of the down kernel: `rw` staged bf16 h rows of one K-half (KH = I / 2), 2 KH + 16 bytes each.
 struct DownLds {

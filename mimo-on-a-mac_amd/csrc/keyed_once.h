@@ -1,9 +1,10 @@
 // A process-lifetime map from a key to one object made on the key's first request (host code).
 //
-// The prefill entry points keep one side stream per (device, caller stream) in such a map: distinct keys get
-// distinct objects, a key gets the same object on every later request, and concurrent first requests of one key
-// from several threads make it once.  Objects are never destroyed (HIP streams and events may still have work
-// queued when the process ends).  Header-only and free of HIP types so a CPU test can exercise it.
+// For objects such as one side stream per (device, caller stream): distinct keys get distinct objects, a key gets the
+// same object on every later request, and concurrent first requests of one key from several threads make it once.
+// Objects are never destroyed (HIP streams and events may still have work queued when the process ends).  No launcher
+// needs one now: every entry point works on its caller's stream alone.  Header-only and free of HIP types so a CPU test
+// can exercise it.
 #pragma once
 #include <map>
 #include <memory>

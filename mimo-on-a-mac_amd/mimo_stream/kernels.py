@@ -158,7 +158,8 @@ def random_bf16(shape, seed, stddev=1.0, device="cuda"):
 
 
 def quantize_fp8_hilo(x):
-    """bf16 [rows, K] -> (hi, hs, lo, ls) uint8 tensors: the activation split the MFMA paths use."""
+    """bf16 [rows, K] -> (hi, hs, lo, ls) uint8 tensors: the two-plane split of activations for
+    block-scaled FP8 MFMAs."""
     _lib.require_cuda(x)
     x = x.to(torch.bfloat16).contiguous()
     rows, K = x.shape
