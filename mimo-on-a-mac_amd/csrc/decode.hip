@@ -31,7 +31,8 @@ struct ExpertsArgs {
   const int32_t *uslot, *urows, *ucnt, *n_unique;
   const float* uw;
   const uint32_t* gidx;
-  uint16_t* h;                              // [Umax, R, I] bf16
+  uint16_t* h;                              // [Umax, R, I] bf16, in the workspace (16-byte pieces are read from it)
+  uint16_t* h_out;                          // the caller's copy, at any address a bf16 can have (optional)
   float* part;                              // [Umax, R, H]
   int round_bf16, zero_pad;
   uint16_t* y;                              // [M, H]
@@ -364,8 +365,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
     const float ut = round_bf16(usum);
     const float sig = sigmoid_bf16(gtf);               // the bf16 sigmoid table's entry for gt, computed in place
     const uint16_t hb = f32_to_bf16(round_bf16(gtf * sig) * ut);
-    if (e_r < cnt || (a.zero_pad && e_r < a.R))   // padding rows (zeros) only for callers that asked for h
-      a.h[((size_t)u * a.R + e_r) * a.I + n0 + e_n] = e_r < cnt ? hb : (uint16_t)0;
+    const size_t at = ((size_t)u * a.R + e_r) * a.I + n0 + e_n;
+    if (e_r < cnt) a.h[at] = hb;
+    if (a.h_out && e_r < a.R) a.h_out[at] = e_r < cnt ? hb : (uint16_t)0;   // its padding rows are zeros
   }
   if (publisher)   // block (0, 0) publishes the full routing for the down kernel
     publish_routes(a, s_inds, s_w, g_uids, g_urows, g_ucnt, g_uw, g_gidx, g_nu, tid);
@@ -708,7 +710,8 @@ int mimo_moe_experts(const uint16_t* x, int M, const mimo_bank* bank, const int3
   a.gate_s = bank->gate_s; a.up_s = bank->up_s; a.down_s = bank->down_s;
   a.H = H; a.I = I; a.R = R; a.Umax = Umax; a.k = k; a.M = M; a.S = bank->n_slots;
   a.uslot = uslot; a.urows = urows; a.ucnt = ucnt; a.n_unique = n_unique; a.uw = uw; a.gidx = gidx;
-  a.h = h_out ? h_out : w.h;
+  a.h = w.h;
+  a.h_out = h_out;
   a.part = part_out ? part_out : w.part;
   a.zero_pad = (h_out || part_out) ? 1 : 0;
   a.y = y;

@@ -216,3 +216,37 @@ def test_fast_selection_equals_slot_table_path(rng, shape, M):
         y, inds, w = blk(xs[:1], return_routes=True)
         oy = ox.gather_m1(x[0], pool, inds.cpu().numpy()[0], w.cpu().numpy()[0])
         assert_bf16_close(bf16_np(y)[0], oy, what="one-row fast selection")
+
+
+@pytest.mark.parametrize("M", [1, 4])
+def test_h_out_at_any_bf16_address(rng, tiny_pool, M):
+    """The caller's copy of h may lie at any multiple of 2 bytes (the ABI asks for no more): y, h and the partials are
+    those of the call that keeps h in the workspace and of one with an aligned copy, and nothing beside h is written."""
+    from mimo_stream import _lib, group_routes
+    from mimo_stream.pools import bank_struct
+    bank, _ = tiny_pool
+    H, I, R, k = 256, 512, 8, 2
+    x = to_dev_bf16(rand_bf16(rng, (M, H)))
+    uids, urows, ucnt, uw, gidx = group_routes(*_routes(rng, M, 8, k), R=R, n_slots=8)
+    U = uids.shape[0]
+    n = U * R * I
+
+    def call(h, part):
+        y = torch.empty((M, H), dtype=torch.bfloat16, device="cuda")
+        ws = torch.zeros(_lib.load().mimo_moe_experts_workspace_size(M, U, R, H, I), dtype=torch.uint8, device="cuda")
+        _lib.call("mimo_moe_experts", _lib.ptr(x), M, bank_struct(bank), _lib.ptr(uids), _lib.ptr(urows),
+                  _lib.ptr(ucnt), _lib.ptr(uw), None, U, R, _lib.ptr(gidx), k, 0, _lib.ptr(y), _lib.ptr(h),
+                  _lib.ptr(part), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(x.device))
+        return y.view(torch.int16)
+
+    y0 = call(None, None)
+    h0 = torch.full((n,), -1, dtype=torch.int16, device="cuda")
+    p0 = torch.empty((U, R, H), dtype=torch.float32, device="cuda")
+    assert torch.equal(call(h0, p0), y0)
+    assert not h0.view(U, R, I)[0, int(ucnt[0]):].any(), "padding rows are zeros"
+    for off in (1, 3, 4):
+        buf = torch.full((n + 16,), -1, dtype=torch.int16, device="cuda")
+        p1 = torch.empty_like(p0)
+        assert torch.equal(call(buf[off:], p1), y0)
+        assert torch.equal(buf[off:off + n], h0) and torch.equal(p1, p0)
+        assert (buf[:off] == -1).all() and (buf[off + n:] == -1).all()
