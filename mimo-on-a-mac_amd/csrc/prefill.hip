@@ -466,15 +466,19 @@ struct PfTiling {
   int wcap, scap, rows;
   bool small;
 };
+static int pf_wide_cap(int64_t P, int S, int rows) {
+  return (int)(P / rows + std::min<int64_t>(S, P / (PF_NARROW_MAX + 1)) + 1);
+}
 static PfTiling pf_tiling(int64_t P, int S) {
   PfTiling t;
   t.small = P <= (int64_t)PF_SMALL_AVG * S;
   t.rows = t.small ? PF_SMALL_ROWS : PF_WIDE_ROWS;
-  t.wcap = (int)(P / t.rows + std::min<int64_t>(S, P / (PF_NARROW_MAX + 1)) + 1);
+  t.wcap = pf_wide_cap(P, S, t.rows);
   t.scap = (int)std::min<int64_t>(S, P);
   return t;
 }
 
+// The need grows with T alone: a workspace sized for the longest chunk holds every shorter one.
 static PrefillWs carve_prefill(Carve& c, int T, int k, int S, int H, int I, int E) {
   PrefillWs w{};
   const size_t P = (size_t)T * k;
@@ -484,15 +488,21 @@ static PrefillWs carve_prefill(Carve& c, int T, int k, int S, int H, int I, int 
   w.perm = c.take<int32_t>(P);
   w.inv = c.take<int32_t>(P);
   w.offsets = c.take<int32_t>(S + 1);
-  w.tiles = c.take<int4>(kTileHead + (size_t)tl.wcap + tl.scap);
+  // with the capacity that tiles of PF_SMALL_ROWS need in either configuration
+  w.tiles = c.take<int4>(kTileHead + (size_t)pf_wide_cap((int64_t)P, S, PF_SMALL_ROWS) + tl.scap);
   if (E > 0) {
-    w.logits = c.take<float>((size_t)(T <= kRlPartsMax ? kRlParts : 1) * T * E);
     w.inds = c.take<int32_t>(P);
     w.w = c.take<float>(P);
     w.slot_inds = c.take<int32_t>(P);
   }
+  // the selection has read the logits before h and Y are written: they share their room
+  Carve over = c;
   w.h = c.take<uint16_t>(P * I);
   w.Y = c.take<uint16_t>(P * H);
+  if (E > 0) {
+    w.logits = over.take<float>((size_t)std::max(T, kRlParts * std::min(T, kRlPartsMax)) * E);
+    c.off = std::max(c.off, over.off);
+  }
   return w;
 }
 

@@ -38,3 +38,31 @@ def test_dispatch_against_oracle(rng, T, k, S):
     want = orr.prefill_dispatch(inds, S)
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g.cpu().numpy(), np.asarray(w))
+
+
+@pytest.mark.parametrize("E,k", [(1024, 1), (300, 5)])
+def test_short_chunk_in_the_longest_chunks_workspace(rng, E, k):
+    """One workspace, sized for 650 tokens and filled with NaN bytes, serves shorter chunks on both sides of the 640
+    tokens at which the logits' form changes.  The logits share the room of h and Y: the outputs are those of the
+    router and the expert entry points called apart."""
+    from mimo_stream import Router, _lib, pools
+    H, I = 256, 128
+    r = Router(H, E, k)
+    r.weight.copy_(to_dev_bf16(rand_bf16(rng, (E, H), 0.05)))
+    weights = pools.random_bank(E, seed=3, hidden=H, inter=I)   # outlives the calls
+    bank = pools.bank_struct(weights)
+    lib = _lib.load()
+    n = lib.mimo_moe_prefill_block_workspace_size(650, E, k, E, H, I)
+    ws = torch.full((n,), 255, dtype=torch.uint8, device="cuda")
+    for T in (640, 641, 9, 650):
+        x = to_dev_bf16(rand_bf16(rng, (T, H)))
+        y, y2 = torch.empty_like(x), torch.empty_like(x)
+        stream = _lib.stream_ptr(x.device)
+        _lib.call("mimo_moe_prefill_block", _lib.ptr(x), T, _lib.ptr(r.weight), _lib.ptr(r.e_score_correction_bias), None,
+                  E, k, bank, _lib.ptr(y), None, None, None, _lib.ptr(ws), n, stream)
+        inds, w = r(x)
+        n2 = lib.mimo_moe_prefill_workspace_size(T, k, E, H, I)
+        ws2 = torch.empty(n2, dtype=torch.uint8, device="cuda")
+        _lib.call("mimo_moe_prefill", _lib.ptr(x), T, _lib.ptr(inds), _lib.ptr(w), k, bank, _lib.ptr(y2), None,
+                  _lib.ptr(ws2), n2, stream)
+        assert torch.isfinite(y).all() and torch.equal(y, y2), T
