@@ -51,8 +51,7 @@ struct ExpertsArgs {
 
 // dword m of a lane's 16 bytes of codes: codes 32 g + 8 m .. of its row
 __device__ __forceinline__ uint32_t word_of(uint4 w, int m) { return m == 0 ? w.x : m == 1 ? w.y : m == 2 ? w.z : w.w; }
-// Whether one of 8 E8M0 bytes is 253 or 254: its weights can reach 2^128, which bf16 cannot hold.  A wave that meets
-// one multiplies with a quarter of every weight (then all fit) and takes its sums times 4.
+// Whether one of 8 E8M0 bytes is 253 or 254 (weights that bf16 cannot hold: the sums are then taken again in parts).
 __device__ __forceinline__ bool has_huge_scale(uint2 v) {
   auto word = [](uint32_t w) {     // bytes ^ 0xFE: 253 -> 3, 254 -> 0; and ^ 0xFD: 253 -> 0
     const uint32_t a = w ^ 0xFEFEFEFEu, b = w ^ 0xFDFDFDFDu;
@@ -298,7 +297,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
   uint32_t any_huge = 0;
 #pragma unroll
   for (int w = 0; w < 4; ++w) any_huge |= s_huge[w];
-  const float fs = any_huge ? 0.25f : 1.0f;   // scale of the weights
+  any_huge = __builtin_amdgcn_readfirstlane(any_huge);
 
   v4f accg = {0.0f, 0.0f, 0.0f, 0.0f}, accu = {0.0f, 0.0f, 0.0f, 0.0f};
   const uint8_t* lrow = lds + i * L.RS + b0;   // this lane's gate scale row (up: + 16 rows)
@@ -313,7 +312,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
     uint32_t gs = *reinterpret_cast<const uint32_t*>(lrow), us = *reinterpret_cast<const uint32_t*>(lrow + 16 * L.RS);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const float scg = e8m0_f32(byte_of(gs, g)) * fs, scu = e8m0_f32(byte_of(us, g)) * fs;
+      const float scg = e8m0_f32(byte_of(gs, g)), scu = e8m0_f32(byte_of(us, g));
       if (s + 1 < NS) {
         gs = *reinterpret_cast<const uint32_t*>(lrow + 4 * (s + 1));
         us = *reinterpret_cast<const uint32_t*>(lrow + 16 * L.RS + 4 * (s + 1));
@@ -340,8 +339,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
     __syncthreads();
     run_pass(c0, accg, accu);
   }
-  accg = accg * (1.0f / fs);
-  accu = accu * (1.0f / fs);
+  if (any_huge) {                  // rare: the sums again in parts, rows and weights straight from memory
+    int ln = lane;
+    asm volatile("" : "+v"(ln));   // nothing of this is kept in registers across the pass above
+    const int gl = ln >> 4, il = ln & 15;
+    int token = __shfl(tok, min(il & 7, cnt - 1), 64);
+    token = (token < 0 || token >= a.M) ? 0 : token;
+    const uint4* xr = reinterpret_cast<const uint4*>(a.x + (size_t)token * a.H + k0) + 4 * gl;
+    const size_t row16 = ((size_t)slot * a.I + n0 + il) * (a.H / 32) + b0 + gl;   // 32-blocks of 16 bytes
+    const uint4 *gp = reinterpret_cast<const uint4*>(a.gate_w) + row16, *up = reinterpret_cast<const uint4*>(a.up_w) + row16;
+    const uint8_t* sp = lds + il * L.RS + b0 + gl;
+    accg = accu = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+      const bool hp = part == 0;
+#pragma unroll 1
+      for (int s = 0; s < NS; ++s) {
+        const uint32_t eg = sp[4 * s], eu = sp[16 * L.RS + 4 * s];
+        const uint4 wg = part_codes(gp[4 * s], eg, hp), wu = part_codes(up[4 * s], eu, hp);
+        const float scg = part_scale(eg, hp), scu = part_scale(eu, hp);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const bf16x8 xm = __builtin_bit_cast(bf16x8, xr[16 * s + m]);
+          accg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(wg, m), scg), xm, accg, 0, 0, 0);
+          accu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(wu, m), scu), xm, accu, 0, 0, 0);
+        }
+      }
+      if (hp) {
+        accg = accg * 4.0f;
+        accu = accu * 4.0f;
+      }
+    }
+  }
   __syncthreads();                 // the activation region is free: the K-range partials go there
   float (*red)[2][32][4] = reinterpret_cast<float (*)[2][32][4]>(lds + L.red);   // [K-range][gate/up][8 g + row][q]
   if (i < 8) {                     // lane (i, g): row i, outputs 4 g + q
@@ -469,7 +498,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t* srow_p = &wsc[wave][i * SRS];
-    const float fs = __ballot(has_huge_scale(sraw)) ? 0.25f : 1.0f;
+    const bool any_huge = __ballot(has_huge_scale(sraw)) != 0;
     // one pass over the staged rows: each activation operand of step s + 1 is read from LDS as step s is done with it
     auto run_pass = [&](int c0, v4f old) __attribute__((always_inline)) {
       const bool avalid = crow >= c0 && crow < min(cnt, c0 + rw);
@@ -480,7 +509,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
       uint32_t bs = srow_p[0];
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        const float sc = e8m0_f32(byte_of(bs, g)) * fs;
+        const float sc = e8m0_f32(byte_of(bs, g));
         if (s + 1 < NS) bs = srow_p[s + 1];
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -502,7 +531,29 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
       run_pass(c0, acc);
     }
-    acc = acc * (1.0f / fs);
+    if (active && any_huge) {            // rare: the sums again in parts, rows and weights straight from memory
+      int ln = lane;
+      asm volatile("" : "+v"(ln));       // nothing of this is kept in registers across the pass above
+      const int gl = ln >> 4, il = ln & 15;
+      const uint4* hr = reinterpret_cast<const uint4*>(a.h + ((size_t)u * a.R + min(il & 7, cnt - 1)) * a.I + kh * L.KH) + 4 * gl;
+      const uint4* wp = reinterpret_cast<const uint4*>(a.down_w) + (bslot + il) * (a.I / 32) + b0 + gl;
+      acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+      for (int part = 0; part < 2; ++part) {
+        const bool hp = part == 0;
+#pragma unroll 1
+        for (int s = 0; s < NS; ++s) {
+          const uint32_t e = byte_of(wsc[wave][il * SRS + s], gl);
+          const uint4 w = part_codes(wp[4 * s], e, hp);
+          const float sc = part_scale(e, hp);
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_bf16x8(word_of(w, m), sc),
+                                                          __builtin_bit_cast(bf16x8, hr[16 * s + m]), acc, 0, 0, 0);
+        }
+        if (hp) acc = acc * 4.0f;
+      }
+    }
     __builtin_amdgcn_wave_barrier();     // the staged rows and scales are read before the next item overwrites them
     if (i < cnt && i < 8 && rbase + i < nr)                      // lane (i, g): row i, outputs 4 g ..
       *reinterpret_cast<v4f*>(&part[(kh * nr + rbase + i) * 16 + 4 * g]) = acc;

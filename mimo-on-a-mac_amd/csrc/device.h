@@ -47,6 +47,15 @@ __device__ __forceinline__ bf16x8 fp4_bf16x8(uint32_t w, float scale) {
   return bf16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
 }
 __device__ __forceinline__ float e8m0_f32(uint32_t byte) { return __uint_as_float(byte << 23); }
+// Scale bytes 253 and 254: sums that meet one are taken again in two parts, first these scale blocks alone at a quarter of
+// their scale (then their weights fit), and on four times those sums all other blocks, exactly as they are.  part_codes
+// clears the codes of the blocks that do not belong to a part.
+__device__ __forceinline__ bool huge_scale(uint32_t byte) { return byte - 253u <= 1u; }
+__device__ __forceinline__ uint4 part_codes(uint4 w, uint32_t byte, bool huge) {
+  const uint32_t keep = huge_scale(byte) == huge ? 0xFFFFFFFFu : 0u;
+  return make_uint4(w.x & keep, w.y & keep, w.z & keep, w.w & keep);
+}
+__device__ __forceinline__ float part_scale(uint32_t byte, bool huge) { return e8m0_f32(byte) * (huge ? 0.25f : 1.0f); }
 
 // ------------------------------------------------------------------ E4M3 (activation hi/lo split)
 // E8M0 exponent X for an E4M3 block with maximum magnitude amax: amax / 2^X in (224, 448].

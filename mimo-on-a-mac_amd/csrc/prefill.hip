@@ -201,117 +201,149 @@ __device__ __forceinline__ void pf_tile(const PrefillArgs& a, uint8_t* pl, int s
   const uint8_t* scr = scl + SB * i + g;
 
   v4f acc[NJ][4];
-  float fs = 1.0f;
-  for (;;) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+  for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc[j][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t big = 2;                                // least of 254 - scale byte (byte 255: NaN whatever the weight)
-    issue_scales(0);
+    for (int t = 0; t < 4; ++t) acc[j][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  uint32_t big = 2;                                  // least of 254 - scale byte (byte 255: NaN whatever the weight)
+  issue_scales(0);
 #pragma unroll
-    for (int u = 0; u < Sh::EARLY; u += Sh::LU) issue_w(u, u);
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      const int token = GATEUP ? tok / a.k : tok;
-      int ln = lane;
-      asm volatile("" : "+v"(ln));                   // kept out of the registers that live across the K loop
+  for (int u = 0; u < Sh::EARLY; u += Sh::LU) issue_w(u, u);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const int token = GATEUP ? tok / a.k : tok;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                   // kept out of the registers that live across the K loop
 #pragma unroll
-      for (int c = 0; c < NJ; ++c) {
-        const int rl = 4 * c + (ln >> 4), r = r0 + rl;
-        const uint32_t row = (uint32_t)__shfl(token, rl, 64) * (uint32_t)(2 * K);
-        const int at = (ln ^ r) & 15;        // 4 m + g of the lane's position
-        a_off[c] = row + (r < nvalid ? 16u * (uint32_t)(4 * (at & 3) + (at >> 2)) : 0u);
-      }
+    for (int c = 0; c < NJ; ++c) {
+      const int rl = 4 * c + (ln >> 4), r = r0 + rl;
+      const uint32_t row = (uint32_t)__shfl(token, rl, 64) * (uint32_t)(2 * K);
+      const int at = (ln ^ r) & 15;        // 4 m + g of the lane's position
+      a_off[c] = row + (r < nvalid ? 16u * (uint32_t)(4 * (at & 3) + (at >> 2)) : 0u);
     }
+  }
 #pragma unroll
-    for (int s = 0; s < AHEAD; ++s)
-      if (s < nK) issue_a(s);
-    if constexpr (GATEUP && !Sh::TAB_LATE) {
+  for (int s = 0; s < AHEAD; ++s)
+    if (s < nK) issue_a(s);
+  if constexpr (GATEUP && !Sh::TAB_LATE) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-        lds_copy16(a.sigtab + PF_SIG_LO + (wave >= 2 ? 32768 : 0), 2048 * (wave & 1) + 1024 * c + 16 * lane,
-                   pl + Sh::TAB + 2048 * wave + 1024 * c);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    for (int c = 0; c < 2; ++c)
+      lds_copy16(a.sigtab + PF_SIG_LO + (wave >= 2 ? 32768 : 0), 2048 * (wave & 1) + 1024 * c + 16 * lane,
+                 pl + Sh::TAB + 2048 * wave + 1024 * c);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = Sh::EARLY; u < D; u += Sh::LU) issue_w(u, u);
-    __builtin_amdgcn_sched_barrier(0);
+  for (int u = Sh::EARLY; u < D; u += Sh::LU) issue_w(u, u);
+  __builtin_amdgcn_sched_barrier(0);
 
-    for (int sb = 0; sb < nK; sb += D) {
+  for (int sb = 0; sb < nK; sb += D) {
 #pragma unroll
-      for (int u = 0; u < D; ++u) {
-        const int s = sb + u;                        // past nK (a last round of fewer than D steps): nothing multiplied
-        // The activation copies of step s have landed once no more than the loads issued after them are in flight:
-        // the weights requested since and, away from the end, AHEAD - 1 steps' copies.
-        if (s + AHEAD <= nK) pf_wait(Sh::newer(u) + (AHEAD - 1) * NJ);
-        else pf_wait(Sh::newer(u));
-        __syncthreads();                             // step s landed everywhere; the slot of step s - 1 is free
-        // the step's weights are waited for here, before any newer copy is issued
-        asm volatile("" : "+v"(braw[u][0]), "+v"(braw[u][1]), "+v"(braw[u][2]), "+v"(braw[u][3])::"memory");
-        if (s + AHEAD < nK) issue_a(s + AHEAD);
-        if (s % PF_SCW == 0 && s + PF_SCW < nK) issue_scales(s / PF_SCW + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        if (s < nK) {
-          const uint8_t* st = pl + (s % Sh::STAGES) * Sh::STAGE;
-          const uint8_t* sp = scr + (s / PF_SCW % 2) * PF_SC + 4 * (s % PF_SCW);
-          float sc[4];
+    for (int u = 0; u < D; ++u) {
+      const int s = sb + u;                        // past nK (a last round of fewer than D steps): nothing multiplied
+      // The activation copies of step s have landed once no more than the loads issued after them are in flight:
+      // the weights requested since and, away from the end, AHEAD - 1 steps' copies.
+      if (s + AHEAD <= nK) pf_wait(Sh::newer(u) + (AHEAD - 1) * NJ);
+      else pf_wait(Sh::newer(u));
+      __syncthreads();                             // step s landed everywhere; the slot of step s - 1 is free
+      // the step's weights are waited for here, before any newer copy is issued
+      asm volatile("" : "+v"(braw[u][0]), "+v"(braw[u][1]), "+v"(braw[u][2]), "+v"(braw[u][3])::"memory");
+      if (s + AHEAD < nK) issue_a(s + AHEAD);
+      if (s % PF_SCW == 0 && s + PF_SCW < nK) issue_scales(s / PF_SCW + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s < nK) {
+        const uint8_t* st = pl + (s % Sh::STAGES) * Sh::STAGE;
+        const uint8_t* sp = scr + (s / PF_SCW % 2) * PF_SC + 4 * (s % PF_SCW);
+        float sc[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t e = sp[16 * SB * t];
+          big = min(big, 254u - e);
+          sc[t] = e8m0_f32(e);
+        }
+        // 4 NJ groups of a route chunk times the 4 weight tiles: a group's activation operand is read PX groups ahead
+        // and the next dword's weights are converted a tile at a time, both while earlier MFMAs run
+        constexpr int G = 4 * NJ, PX = NJ == 1 ? 1 : 3;
+        auto read_x = [&](int f) { return *reinterpret_cast<const bf16x8*>(st + (aoff ^ (64 * (f / NJ))) + 4096 * (f % NJ)); };
+        bf16x8 X[PX + 1], W[Sh::WB][4];
+#pragma unroll
+        for (int f = 0; f < PX; ++f) X[f] = read_x(f);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) W[0][t] = fp4_bf16x8(braw[u][t][0], sc[t]);
+#pragma unroll
+        for (int f = 0; f < G; ++f) {
+          const int m = f / NJ, j = f % NJ;
+          __builtin_amdgcn_sched_barrier(0);
+          if (f + PX < G) X[(f + PX) & PX] = read_x(f + PX);
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            const uint32_t e = sp[16 * SB * t];
-            big = min(big, 254u - e);
-            sc[t] = e8m0_f32(e) * fs;
+            if (Sh::WB == 2 && m < 3 && t * NJ / 4 == j) W[(m + 1) & 1][t] = fp4_bf16x8(braw[u][t][m + 1], sc[t]);
+            if (Sh::WB == 1 && m > 0 && j == 0) W[0][t] = fp4_bf16x8(braw[u][t][m], sc[t]);
           }
-          // 4 NJ groups of a route chunk times the 4 weight tiles: a group's activation operand is read PX groups ahead
-          // and the next dword's weights are converted a tile at a time, both while earlier MFMAs run
-          constexpr int G = 4 * NJ, PX = NJ == 1 ? 1 : 3;
-          auto read_x = [&](int f) { return *reinterpret_cast<const bf16x8*>(st + (aoff ^ (64 * (f / NJ))) + 4096 * (f % NJ)); };
-          bf16x8 X[PX + 1], W[Sh::WB][4];
 #pragma unroll
-          for (int f = 0; f < PX; ++f) X[f] = read_x(f);
+          for (int t = 0; t < 4; ++t)
+            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[m % Sh::WB][t], X[f & PX], acc[j][t], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (u % Sh::LU == Sh::LU - 1) issue_w(u - Sh::LU + 1, s + D - Sh::LU + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // Scale bytes 253 and 254 (weights that bf16 cannot hold): the tile's sums are taken again in parts, rows, weights and
+  // scales straight from memory
+  const bool over = __ballot(big <= 1u) != 0;
+  uint32_t* flag = reinterpret_cast<uint32_t*>(pl + Sh::LDS - 16);
+  wait_vm_all();
+  __syncthreads();                                   // every wave is done with the ring and the scales
+  if (lane == 0) flag[wave] = over ? 1u : 0u;
+  if constexpr (GATEUP && Sh::TAB_LATE) {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) W[0][t] = fp4_bf16x8(braw[u][t][0], sc[t]);
+    for (int c = 0; c < 2; ++c)
+      lds_copy16(a.sigtab + PF_SIG_LO + (wave >= 2 ? 32768 : 0), 2048 * (wave & 1) + 1024 * c + 16 * lane,
+                 pl + Sh::TAB + 2048 * wave + 1024 * c);
+    wait_vm_all();
+  }
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(flag[0] | flag[1] | flag[2] | flag[3])) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                     // nothing of this is kept in registers across the K loop
+    const int gl = ln >> 4, il = ln & 15;
+    uint32_t xrow[NJ];                               // byte offsets of the lane's routes 16 j + i, codes 32 g ..
 #pragma unroll
-          for (int f = 0; f < G; ++f) {
-            const int m = f / NJ, j = f % NJ;
-            __builtin_amdgcn_sched_barrier(0);
-            if (f + PX < G) X[(f + PX) & PX] = read_x(f + PX);
+    for (int j = 0; j < NJ; ++j) {
+      const int p = beg + (PF_UNIT * j + il < nvalid ? PF_UNIT * j + il : 0);
+      xrow[j] = (uint32_t)(GATEUP ? a.perm[p] / a.k : p) * (uint32_t)(2 * K) + 64u * gl;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              if (Sh::WB == 2 && m < 3 && t * NJ / 4 == j) W[(m + 1) & 1][t] = fp4_bf16x8(braw[u][t][m + 1], sc[t]);
-              if (Sh::WB == 1 && m > 0 && j == 0) W[0][t] = fp4_bf16x8(braw[u][t][m], sc[t]);
-            }
+      for (int t = 0; t < 4; ++t) acc[j][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+      const bool hp = part == 0;
+#pragma unroll 1
+      for (int s = 0; s < nK; ++s)
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-              acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[m % Sh::WB][t], X[f & PX], acc[j][t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t e = (t < 2 ? s0p : s1p)[out_row(t, il) * KS + 4 * s + gl];
+          const uint8_t* wp = (t < 2 ? w0 : w1) + (size_t)out_row(t, il) * RB + 16 * gl + 64 * s;
+          const float sc = part_scale(e, hp);
+#pragma unroll 1
+          for (int m = 0; m < 4; ++m) {
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(wp + 4 * m);
+            const bf16x8 W = fp4_bf16x8(huge_scale(e) == hp ? w : 0u, sc);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  W, *reinterpret_cast<const bf16x8*>(act + xrow[j] + 256u * s + 16 * m), acc[j][t], 0, 0, 0);
           }
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (u % Sh::LU == Sh::LU - 1) issue_w(u - Sh::LU + 1, s + D - Sh::LU + 1);
-        __builtin_amdgcn_sched_barrier(0);
+      if (hp) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[j][t] = acc[j][t] * 4.0f;
       }
     }
-    // Scale bytes 253 and 254 make weights of 2^128 and more, which bf16 cannot hold: the tile is run again with every
-    // weight a quarter of its value (then all fit) and the sums are multiplied by 4.
-    const bool over = __ballot(big <= 1u) != 0;
-    uint32_t* flag = reinterpret_cast<uint32_t*>(pl + Sh::LDS - 16);
-    wait_vm_all();
-    __syncthreads();                                 // every wave is done with the ring and the scales
-    if (lane == 0) flag[wave] = over ? 1u : 0u;
-    if constexpr (GATEUP && Sh::TAB_LATE) {
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        lds_copy16(a.sigtab + PF_SIG_LO + (wave >= 2 ? 32768 : 0), 2048 * (wave & 1) + 1024 * c + 16 * lane,
-                   pl + Sh::TAB + 2048 * wave + 1024 * c);
-      wait_vm_all();
-    }
-    __syncthreads();
-    const uint32_t any = flag[0] | flag[1] | flag[2] | flag[3];
-    if (__builtin_amdgcn_readfirstlane(any) == 0 || fs != 1.0f) break;
-    fs = 0.25f;
-    __syncthreads();                                 // the flags are read before the next run's scales arrive
   }
-  const float back = fs == 1.0f ? 1.0f : 4.0f;
 
   // epilogue: lane (i, g) holds route 16 j + i at outputs 8 g .. (GATEUP) or 16 g .. of the wave
   if constexpr (GATEUP) {
@@ -323,10 +355,10 @@ __device__ __forceinline__ void pf_tile(const PrefillArgs& a, uint8_t* pl, int s
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint16_t gt = f32_to_bf16(acc[j][b][q] * back);
+          const uint16_t gt = f32_to_bf16(acc[j][b][q]);
           const int mag = min(max((int)(gt & 0x7FFF), PF_SIG_LO), PF_SIG_LO + PF_SIG_N - 1) - PF_SIG_LO;
           const float sig = bf16_to_f32(tab[mag + ((gt & 0x8000) ? PF_SIG_N : 0)]);
-          hv[4 * b + q] = round_bf16(bf16_to_f32(gt) * sig) * round_bf16(acc[j][2 + b][q] * back);
+          hv[4 * b + q] = round_bf16(bf16_to_f32(gt) * sig) * round_bf16(acc[j][2 + b][q]);
         }
       const int r = PF_UNIT * j + i;
       if (r < nvalid)
@@ -341,7 +373,7 @@ __device__ __forceinline__ void pf_tile(const PrefillArgs& a, uint8_t* pl, int s
       uint4* dst = reinterpret_cast<uint4*>(a.Y + (size_t)(beg + r) * a.H + n0 + 64 * wave + 16 * g);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const v4f p = acc[j][2 * b] * back, q = acc[j][2 * b + 1] * back;
+        const v4f p = acc[j][2 * b], q = acc[j][2 * b + 1];
         dst[b] = make_uint4(pf_pack2(p[0], p[1]), pf_pack2(p[2], p[3]), pf_pack2(q[0], q[1]), pf_pack2(q[2], q[3]));
       }
     }
