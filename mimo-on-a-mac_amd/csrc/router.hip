@@ -6,6 +6,8 @@
 // (sigmoid + bias), ties to the lower expert id, NaN keys last; weights are renormalised with a sequential
 // fp32 sum in that order.  Everything here is integer or exactly specified fp32/fp64 arithmetic, so routes
 // and permutations are bit-exact against the oracle given identical logits.
+#include <algorithm>
+
 #include "device.h"
 #include "host.h"
 #include "layer.h"
@@ -415,6 +417,9 @@ __global__ void group_routes_kernel(const int32_t* inds, const float* scores, co
 // ------------------------------------------------------------------ prefill dispatch (stable counting sort)
 constexpr int DISPATCH_CHUNK = 1024;
 constexpr int kCountChunks = 16;      // up to so many chunks every placement block counts all of them itself
+// Counters per slot there: lanes that count one slot at once wait for each other only within a copy (16,384 routes on
+// two slots: 21.0 us with one counter per slot)
+__host__ __device__ constexpr int count_copies(int n_slots) { return n_slots <= 512 ? 16 : 8; }
 
 // slot ids outside [0, n_slots) are counted as slot 0 and flagged in *status (never indexed out of bounds)
 __device__ __forceinline__ int checked_slot(const int32_t* slots, int i, int n_slots, int32_t* status) {
@@ -453,7 +458,7 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
                                                                    TileSpec spec, int4* __restrict__ tiles,
                                                                    int32_t* __restrict__ perm, int32_t* __restrict__ inv,
                                                                    int32_t* status, bool zero_status) {
-  extern __shared__ int dsp[];                   // base[n_slots], then wc[16 waves][n_slots] (counts <= 64)
+  extern __shared__ __align__(16) int dsp[];     // base[n_slots], then wc[16 waves][n_slots] (counts <= 64)
   int* base = dsp;
   uint16_t* wc = reinterpret_cast<uint16_t*>(dsp + n_slots);
   __shared__ int wsum[4][16];
@@ -462,8 +467,11 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   int c = 0, pre = 0;
   int mine = -1;                                 // COUNT: the thread's route of this chunk
   if constexpr (COUNT) {
-    // counts in the place of base (all chunks) and of wc (the earlier chunks, n_slots words)
-    int* early = dsp + n_slots;
+    // counters in the place of base and wc: all chunks in the low half, the earlier ones in the high (at most 2^14 each);
+    // copy c of slot s at C s + c
+    static_assert(kCountChunks * DISPATCH_CHUNK < 1 << 16, "16-bit counts");
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(dsp);
+    const int C = count_copies(n_slots);
     __shared__ int s_bad;
     int sl[kCountChunks];
 #pragma unroll
@@ -471,7 +479,7 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
       const int i = b * DISPATCH_CHUNK + tid;
       sl[b] = b < nchunks && i < n ? slots[i] : -1;
     }
-    for (int i = tid; i < 2 * n_slots; i += blockDim.x) dsp[i] = 0;
+    for (int i = tid; i < C * n_slots / 4; i += blockDim.x) reinterpret_cast<uint4*>(cnt)[i] = make_uint4(0, 0, 0, 0);
     if (tid == 0) s_bad = 0;
     __syncthreads();
 #pragma unroll
@@ -483,15 +491,16 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
           s_bad = 1;
           s = 0;
         }
-        atomicAdd(&base[s], 1);                  // integer counts: order independent
-        if (b < blk) atomicAdd(&early[s], 1);
+        atomicAdd(&cnt[C * s + (tid & (C - 1))], b < blk ? 0x10001u : 1u);   // integer counts: order independent
         if (b == blk) mine = s;
       }
     }
     __syncthreads();
     if (tid < n_slots) {
-      c = base[tid];
-      pre = early[tid];
+      uint32_t v = 0;
+      for (int j = 0; j < C; ++j) v += cnt[C * tid + ((j ^ tid) & (C - 1))];   // the lanes' reads spread over the banks
+      c = (int)(v & 0xFFFFu);
+      pre = (int)(v >> 16);
     }
     if (status && blk == 0 && tid == 0) {
       if (zero_status) *status = s_bad ? MIMO_ERR_SLOT : MIMO_OK;
@@ -588,8 +597,9 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
   }
 }
 
-// Up to kCountChunks chunks one launch, which counts in every block; more take a histogram launch first (8 blocks
-// counting 8 chunks each cost less than the launch; the counting grows with the square of the chunks).
+// Up to kCountChunks chunks one launch, which counts in every block; more take a histogram launch first.  At 16 chunks
+// (16,384 routes) one launch takes 7.9 us and two 10.4 with 256 slots, spread evenly or all on two slots; 8.7 and 10.2
+// with 1024.  The counting of all chunks in every block grows with the square of the chunks.
 int launch_dispatch(const int32_t* slots, int n, int n_slots, int32_t* hist, int32_t* perm, int32_t* offsets,
                     int32_t* inv, const TileSpec* spec, int4* tiles, int32_t* status, bool zero_status, hipStream_t st) {
   int nchunks = (n + DISPATCH_CHUNK - 1) / DISPATCH_CHUNK;
@@ -598,7 +608,8 @@ int launch_dispatch(const int32_t* slots, int n, int n_slots, int32_t* hist, int
   const TileSpec none{0, 1, 0};
   const size_t lds = n_slots * (sizeof(int) + 16 * sizeof(uint16_t));
   if (nchunks <= kCountChunks) {
-    dispatch_scan_place_kernel<true><<<nchunks, 1024, lds, st>>>(slots, n, nullptr, nchunks, n_slots, offsets,
+    const size_t lds_count = std::max(lds, n_slots * count_copies(n_slots) * sizeof(uint32_t));
+    dispatch_scan_place_kernel<true><<<nchunks, 1024, lds_count, st>>>(slots, n, nullptr, nchunks, n_slots, offsets,
                                                                  spec ? *spec : none, spec ? tiles : nullptr, perm, inv,
                                                                  status, zero_status);
     return check_launch("prefill dispatch");

@@ -66,3 +66,18 @@ def test_short_chunk_in_the_longest_chunks_workspace(rng, E, k):
         _lib.call("mimo_moe_prefill", _lib.ptr(x), T, _lib.ptr(inds), _lib.ptr(w), k, bank, _lib.ptr(y2), None,
                   _lib.ptr(ws2), n2, stream)
         assert torch.isfinite(y).all() and torch.equal(y, y2), T
+
+
+@pytest.mark.parametrize("T,k,S", [(2048, 8, 1), (2048, 8, 2), (2047, 8, 3), (2048, 8, 512), (2048, 8, 513), (2048, 8, 1024),
+                                   (1, 1, 1024), (2049, 8, 2)])
+@pytest.mark.parametrize("slots", ["one", "last two"])
+def test_dispatch_of_crowded_slots(T, k, S, slots):
+    """Every route on one slot or two: the counters' largest counts, at the slot counts where their copies change."""
+    from mimo_stream import prefill_dispatch
+    inds = np.full((T, k), S - 1, np.int32)
+    if slots == "last two":
+        inds[::3] = max(S - 2, 0)
+    got = prefill_dispatch(torch.from_numpy(inds).cuda(), S)
+    want = orr.prefill_dispatch(inds, S)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g.cpu().numpy(), np.asarray(w))
