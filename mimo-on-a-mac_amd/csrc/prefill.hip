@@ -58,6 +58,11 @@ constexpr int PF_WIDE_ROWS = 128;
 // tokens: 763 us, 733 with 48).
 constexpr int PF_SMALL_AVG = 24;
 constexpr int PF_SMALL_ROWS = 64;
+// It also runs when the wide tiles are fewer blocks than CUs (full tiles times gate/up output blocks): half the rows make
+// twice the blocks.  H 4096, I 384, 64 slots: 800 tokens on 6 slots (112 blocks) 111 us a layer against 132, spread over
+// all 134 against 129, 1700 spread (239) 200 against 215; H 7168, I 256, 32 slots, 800 tokens (50) 144 against 177; H 256,
+// I 2048, 16 slots, 800 tokens (200) 53 against 63.  Above: H 768, I 384, 12 slots, 6000 tokens (422) 97 against 89.
+constexpr int PF_FEW_BLOCKS = 256;
 constexpr int PF_UNIT = 16;                          // routes per MFMA chunk
 constexpr int PF_ROWS = 256;                         // weight rows per block
 // the part of the bf16 sigmoid table that is not constant: |x| in [2^-9, 128) (below, 0.5; above, 0 or 1)
@@ -501,9 +506,9 @@ struct PfTiling {
 static int pf_wide_cap(int64_t P, int S, int rows) {
   return (int)(P / rows + std::min<int64_t>(S, P / (PF_NARROW_MAX + 1)) + 1);
 }
-static PfTiling pf_tiling(int64_t P, int S) {
+static PfTiling pf_tiling(int64_t P, int S, int I) {
   PfTiling t;
-  t.small = P <= (int64_t)PF_SMALL_AVG * S;
+  t.small = P <= (int64_t)PF_SMALL_AVG * S || P * I < (int64_t)PF_FEW_BLOCKS * PF_WIDE_ROWS * (PF_ROWS / 2);
   t.rows = t.small ? PF_SMALL_ROWS : PF_WIDE_ROWS;
   t.wcap = pf_wide_cap(P, S, t.rows);
   t.scap = (int)std::min<int64_t>(S, P);
@@ -514,7 +519,7 @@ static PfTiling pf_tiling(int64_t P, int S) {
 static PrefillWs carve_prefill(Carve& c, int T, int k, int S, int H, int I, int E) {
   PrefillWs w{};
   const size_t P = (size_t)T * k;
-  const PfTiling tl = pf_tiling((int64_t)P, S);
+  const PfTiling tl = pf_tiling((int64_t)P, S, I);
   w.status = c.take<int32_t>(1);
   w.hist = reinterpret_cast<int32_t*>(c.take<char>(dispatch_workspace((int)P, S)));
   w.perm = c.take<int32_t>(P);
@@ -561,7 +566,7 @@ static int run_prefill(const uint16_t* x, int T, const int32_t* slot_inds, const
   int err;
   const uint16_t* sig = sigtab_device(&err);
   if (!sig) return err;
-  const PfTiling tl = pf_tiling(P, S);
+  const PfTiling tl = pf_tiling(P, S, I);
   const TileSpec spec{PF_NARROW_MAX, tl.rows, tl.wcap};
   int rc = launch_dispatch(slot_inds, P, S, ws.hist, ws.perm, ws.offsets, ws.inv, &spec, ws.tiles, ws.status,
                            zero_status, st);

@@ -563,14 +563,14 @@ __global__ void __launch_bounds__(1024) dispatch_scan_place_kernel(const int32_t
         if (tiles) tiles[0] = make_int4(v1, v2, 0, 0);
       }
       if (nw) {
-        int total = 0;
+        uint32_t total = 0;                      // below 2^27 (fewer than 2^30 routes): eighths in 32 bits
         for (int w = 0; w < 16; ++w) total += wsum[3][w];
         for (int q = 0; q < nw; ++q) {
           tiles[kTileHead + e1 + q] = make_int4(tid, e0 + spec.wide_rows * q, e0 + min(spec.wide_rows * (q + 1), c), 0);
           // the shares that start within this tile: 8 cum <= total x < 8 (cum + cost)
-          const int cum = v3 - cost + full * q, tc = q == nw - 1 ? last : full;
-          for (int x = (int)((8ll * cum + total - 1) / total); x < 8 && (int64_t)total * x < 8ll * (cum + tc); ++x)
-            tiles[1 + x] = make_int4(e1 + q, (int)((int64_t)total * x - 8ll * cum), tc, 0);
+          const uint32_t cum = v3 - cost + full * q, tc = q == nw - 1 ? last : full;
+          for (uint32_t x = (8 * cum + total - 1) / total; x < 8 && total * x < 8 * (cum + tc); ++x)
+            tiles[1 + x] = make_int4(e1 + q, (int)(total * x - 8 * cum), (int)tc, 0);
         }
       }
       if (ns) tiles[kTileHead + spec.wcap + e2] = make_int4(tid, e0, e0 + c, 0);

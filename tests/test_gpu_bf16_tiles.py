@@ -65,6 +65,35 @@ def test_prefill_scales_of_unaligned_pools(rng):
         np.testing.assert_array_equal(y, y2)
 
 
+def _many_blocks(I):
+    """MANY and one more slot, crowded enough that the wide tiles are as many blocks as the chip has CUs (256 blocks of
+    128 routes times 128 outputs of I); with fewer, or up to 24 routes a slot, the streaming configuration runs."""
+    return MANY + [256 * 128 * 128 // I + 1 - sum(MANY)]
+
+
+@pytest.mark.parametrize("H,I", [(256, 128), (512, 640), (768, 384), (1024, 1152), (256, 4224)])
+def test_prefill_wide_tile_edges(rng, H, I):
+    """The tile edges in the wide configuration, and its scales from pools whose rows cannot be copied 16 bytes at a
+    time: the same bits."""
+    from mimo_stream import MoEBlock
+    counts = _many_blocks(I)
+    blk, bank = _block(H, I, len(counts), seed=H + I)
+    state = rng.bit_generator.state
+    y, oy = _prefill(rng, blk, bank, counts)
+    assert_bf16_close(y, oy, what=f"H={H} I={I}")
+    moved = dict(bank)
+    for p in ("gate_s", "up_s", "down_s"):
+        moved[p] = torch.empty(bank[p].numel() + 4, dtype=torch.uint8, device="cuda")[4:].view(bank[p].shape)
+        moved[p].copy_(bank[p])
+    rng.bit_generator.state = state
+    inds = np.repeat(np.arange(len(counts)), counts)[:, None].astype(np.int32)      # the same rows, routes and weights
+    rng.shuffle(inds)
+    x = rand_bf16(rng, (len(inds), H))
+    w = (0.5 + rng.random((len(inds), 1))).astype(np.float32)
+    y2 = MoEBlock(blk.router, moved)._moe_prefill(to_dev_bf16(x), torch.from_numpy(inds).cuda(), torch.from_numpy(w).cuda())
+    np.testing.assert_array_equal(y, bf16_np(y2))
+
+
 @pytest.mark.parametrize("M,same", [(3, 3), (4, 4), (5, 5), (8, 1), (8, 4), (8, 5), (8, 8)])
 def test_decode_rows_per_expert(rng, M, same):
     """`same` of the M rows share their first expert; more than four rows of one expert take a second pass."""

@@ -4,8 +4,8 @@ not fit bf16) beside 0 and 1 (2^-127 and 2^-126).
 Every other block of 32 codes meets activations of about 2^122 under small scales, the ones between activations of about
 2^-126 under large ones, so both add sums of ordinary size to every result and each must come out at its own scale.
 Against the oracle at the parity bar, each kind of weight row held to its own magnitude; decode through the fused block
-(1 to 5 rows) and through moe_experts (up to 8 rows of one expert, more than are staged at once), prefill in both of its
-tile configurations."""
+(1 to 8 rows, up to 8 of one expert, more than are staged at once), prefill in both of its tile configurations (the wide
+one from 2731 rows)."""
 import numpy as np
 import pytest
 import torch
@@ -83,7 +83,7 @@ def _check(case, got, ref, what):
 
 
 @pytest.mark.parametrize("case", ["gate_up", "down"])
-@pytest.mark.parametrize("T", [1, 2, 3, 5, 8, 20, 100, 150])
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 8, 20, 100, 150, 2750])
 def test_block(rng, case, T):
     blk, bank = _block(rng, seed=71)
     {"gate_up": _gate_up, "down": _down}[case](rng, bank)
