@@ -5,7 +5,6 @@
 
 namespace mimo {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -177,30 +176,6 @@ __device__ __forceinline__ void quant_block_fp8_hilo(const float* v, uint32_t* h
 }
 
 // ------------------------------------------------------------------ wave reductions (wave64)
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    uint64_t w = __shfl_xor(v, o, 64);
-    v = w > v ? w : v;
-  }
-  return v;
-}
-// max over groups of `width` consecutive lanes (width a power of two <= 64)
-__device__ __forceinline__ float group_max(float v, int width) {
-  for (int o = width >> 1; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
 // wave64 sum through DPP row operations (xor 1, xor 2, half-row and row mirrors, then row_bcast15 / 31 into
 // rows 1-3); the total is read from lane 63 and returned to every lane
 __device__ __forceinline__ float dpp_sum_f32(float v) {
@@ -275,12 +250,6 @@ __device__ __forceinline__ void lds_copy4(const void* gbase, uint32_t voff, cons
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(b), "s"(m)
                : "memory", "m0");
 }
-// 16 bytes per lane global -> VGPRs, not tracked by the compiler's wait counting: the caller waits for it with
-// an explicit s_waitcnt before any use (and pins the use below that wait)
-__device__ __forceinline__ void gload16(v4i& dst, const void* gbase, uint32_t voff) {
-  const uint64_t b = uniform_u64((uint64_t)gbase);
-  asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %1, %2" : "=v"(dst) : "v"(voff), "s"(b) : "memory");
-}
 #pragma clang diagnostic pop
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima): every global load of the wave has landed,
 // including the global -> LDS copies above
@@ -293,8 +262,5 @@ __device__ __forceinline__ void wait_vm_keep() {
   static_assert(N >= 0 && N < 64, "vmcnt holds 6 bits");
   __builtin_amdgcn_s_waitcnt(vm_keep(N));
 }
-
-// ------------------------------------------------------------------ misc
-__device__ __forceinline__ uint32_t load_u8x4(const uint8_t* p) { return *(const uint32_t*)p; }
 
 }  // namespace mimo
