@@ -799,7 +799,7 @@ def main():
     out = {
         "metric": METRIC, "value": head["GBps"], "unit": "GB/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": head["ms_per_layer"], "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "mxfp4 x bf16 -> fp32 (block-scaled fp8/fp4 MFMA)", "data": "synthetic",
+        "vs_baseline": None, "dtype": "mxfp4 x bf16 -> fp32 (bf16 MFMA)", "data": "synthetic",
         "config": {"workload": "MiMo-V2.6-Flash MoE layer decode, 1 row: router 4096->256 bf16, top-8, 256 "
                                "resident MXFP4 experts (I=2048, group 32), SwiGLU, fixed-order combine",
                    "hidden": H, "experts": E, "top_k": K, "intermediate": I, "rows": 1,
