@@ -10,7 +10,7 @@ e8m0(s) = 2^(s-127) with s=0 -> 2^-127 and s=255 -> NaN.
 The quantisers here are written from the OCP specification (the reference's mx.quantize is third-party MLX and only makes test
 data: both sides of every parity check consume the same packed bytes).  quantize_mxfp4 follows the OCP
 Microscaling v1.0 rule (shared exponent floor(log2(amax)) - 2, round-to-nearest-even onto the E2M1 grid,
-saturate at 6).  quantize_fp8_hilo is the activation split used by the block-scaled MFMA paths: a bf16 value
+saturate at 6).  quantize_fp8_hilo is the two-plane activation split for block-scaled FP8 MFMAs: a bf16 value
 x is written as hi + lo, both E4M3 with their own E8M0 block scale, which represents every bf16 value of a
 block exactly unless it sits more than ~14 binades below the block maximum.
 """

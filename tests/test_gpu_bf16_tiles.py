@@ -1,8 +1,8 @@
 """The expert products on bf16 MFMA at the edges of their tilings, against the oracle.
 
 Prefill: routes per slot at and beside every chunk count a row tile can have (1 to 128 routes, then a second tile), in
-the kernel of few routes per slot and in the one of many, at reduction lengths of 1 to 32 K-steps that do and do not
-fill a round of the K loop, with scale rows that can and cannot be copied 16 bytes at a time.  Decode: rows per expert
+the streaming configuration (few routes per slot, or few blocks) and in the wide one, at reduction lengths of 1 to 33
+K-steps that do and do not fill a round of the K loop, with scale rows that can and cannot be copied 16 bytes at a time.  Decode: rows per expert
 at and beside the number staged at once.  Both: E8M0 bytes 253 and 254, whose weights (up to 6 * 2^127) do not fit
 bf16.  The bar is the parity tests' own."""
 import numpy as np

@@ -191,9 +191,8 @@ def test_workspace_reuse_across_shapes(rng, tiny_pool, mimo_pool):
 @pytest.mark.parametrize("shape", ["mimo", "tiny"])
 def test_fast_selection_equals_slot_table_path(rng, shape, M):
     """One or two rows with expert ids as slots take the fast path: each gate/up block finds its expert from the
-    threshold searches alone, blocks cover 16 outputs and write h in bf16, and the down kernel splits h into the
-    hi/lo planes.  An explicit identity slot table takes the general routed path (full selection and grouping in
-    every block, 32-output blocks splitting h themselves).  Both give the same bits, with and without the residual
+    threshold searches alone.  An explicit identity slot table takes the general routed path (full selection and
+    grouping in every block).  Both give the same bits, with and without the residual
     of the layer step, over many steps in a row, and match the oracle."""
     from mimo_stream import MoEBlock, MoELayer, pools
     H, I, E, k = (4096, 2048, 256, 8) if shape == "mimo" else (256, 512, 8, 2)

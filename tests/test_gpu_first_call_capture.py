@@ -1,8 +1,8 @@
 """HIP graph capture of a process's first library call: a prefill.
 
-The first prefill of a process looks up the sigmoid table (constant data in the code object), sets the GEMM
-kernels' LDS attribute and creates the side stream of its caller stream.  None of that is stream work, so the
-call may be the first one of a process and run under stream capture.  The case runs in a child process whose
+The first prefill of a process looks up the sigmoid table (constant data in the code object) and sets the GEMM
+kernels' LDS attribute.  None of that is stream work, so the call may be the first one of a process and run under
+stream capture.  The case runs in a child process whose
 inputs are made by torch alone (no library call before the captured one); the graph is replayed three times with
 eager library calls and synchronisations between the replays, and every replay must equal the eager result bit
 for bit."""
@@ -64,8 +64,7 @@ def test_first_prefill_of_a_process_captured():
     run_child(PREFILL_CHILD, "PREFILL_FIRST_CALL_OK")
 
 
-# More caller streams than the library keeps side streams for (64 per device): the prefills on the later streams
-# run both tile launches on their own stream and give the same bits.
+# Many caller streams: nothing is kept per stream, and every prefill gives the same bits.
 MANY_STREAMS_CHILD = CHILD_COMMON + r"""
 H, I, E, k, T = 1024, 512, 64, 8, 300
 bank = torch_bank(E, H, I)

@@ -1,6 +1,6 @@
-"""HIP graph capture of the MoE block: a prefill chunk (narrow tiles on the library's side stream, wide tiles
-on the caller's stream, joined by events) and a one-row decode step, captured once and replayed several times
-with eager work and synchronisations between replays; every replay must equal the eager result bit for bit."""
+"""HIP graph capture of the MoE block: a prefill chunk (popular slots in several row tiles, rarely chosen ones in one
+each, all on the caller's stream) and a one-row decode step, captured once and replayed several times with eager work
+and synchronisations between replays; every replay must equal the eager result bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -46,9 +46,8 @@ def test_prefill_and_decode_graph_replays_match_eager(rng):
 
 
 def test_prefill_from_two_host_threads_on_two_streams(rng):
-    """Two host threads run prefills of different inputs on two streams of the same device at once: the narrow
-    tiles of both share the library's side stream, and each call's fork and join must wait on its own stream's
-    work only, so both results equal the single-threaded ones."""
+    """Two host threads run prefills of different inputs on two streams of the same device at once, each with its own
+    stream's workspace: nothing is shared between the calls, so both results equal the single-threaded ones."""
     import threading
     from mimo_stream import pools, Router, MoEBlock
     H, I, E, k = 4096, 2048, 64, 8

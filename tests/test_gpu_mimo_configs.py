@@ -253,7 +253,7 @@ def test_prefill_zipf_every_token(stack, T):
 @pytest.mark.parametrize("profile_row", [0, 43])
 def test_prefill_measured_popularity_every_token(stack, profile_row):
     """2048 tokens routed with the measured popularity of MiMo layers 1 and 44 (the reference's expert profile):
-    the prefill tiling's mix of wide and narrow tiles under real routing, every token and 64 full combines."""
+    the prefill tiling's mix of many-route and few-route tiles under real routing, every token and 64 full combines."""
     rng = np.random.default_rng(_run_seed() + 7 * profile_row)
     inds = _profile_routes(rng, 2048, profile_row)
     _prefill_every_token(rng, stack[3], 2048, inds, f" (MiMo layer {profile_row + 1} popularity)", 64)

@@ -4,15 +4,14 @@ distinct-expert path with its intermediates, and the prefill block), against the
 Reference semantics (engine/mimo_stream/kernels.py:24-29, :59-77, :113-119): scale byte 0 is 2^-127 and byte 255
 is NaN, applied to each 32-group's partial dot product, so a NaN scale makes that output NaN for every row routed
 to the expert (gate/up: the whole h column, and through the down projection every output of those rows; down:
-that output).  The block-scaled MFMA takes the same E8M0 bytes (v_mfma_scale_f32_16x16x128_f8f6f4): byte 255
-gives NaN products, byte 0 products of at most 6 * 448 * 2^-127 per element, which no bf16 result can see.
+that output).  The weights' conversion to bf16 takes the same E8M0 bytes: byte 255 gives NaN weights, byte 0 weights of
+at most 6 * 2^-127, which bf16 holds exactly (as subnormals) and the MFMA multiplies as they are.
 
-Non-finite activations: a NaN element makes every dot product of its row NaN, in the reference and here (the
-hi/lo split codes it as the E4M3 NaN).  An infinite element gives the reference +-inf or NaN per output of the
-gate/up products, depending on the sign and zeroness of the weight it meets, and from there NaN in h and in every
-output of the row's down projection (h holds infinities and NaNs; the down weights hold zero codes).  Here the
-split codes an infinity as the E4M3 NaN too (E4M3 has no infinity), so h is NaN where the reference has +-inf
-or NaN; the block output y is NaN at exactly the reference's positions.  The router sees the same +-inf / NaN
+Non-finite activations: a NaN element makes every dot product of its row NaN, in the reference and here.  An infinite
+element gives +-inf or NaN per output of the gate/up products, depending on the sign and zeroness of the weight it
+meets, in the reference and here alike (the bf16 activations are multiplied as they are), and from there NaN in every
+output of the row's down projection (h holds infinities and NaNs; the down weights hold zero codes): the block output y
+is NaN at exactly the reference's positions.  The router sees the same +-inf / NaN
 logits as the reference (IEEE fp32 arithmetic, NaN-insensitive to order) and selects bit-exactly.  Rows without
 a non-finite element are unaffected and meet the usual tolerance."""
 import numpy as np

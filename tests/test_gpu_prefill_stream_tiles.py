@@ -1,6 +1,7 @@
 """The prefill GEMMs' streaming configuration (few routes per slot) cuts popular slots into tiles of up to 64 routes: slots
 at and beside each of its chunk counts and tile ends, at the average on both sides of the line to the other
-configuration, against the oracle."""
+configuration (which needs 256 blocks of 128 routes times 128 outputs as well: only I = 5376 passes the line), against
+the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -14,7 +15,7 @@ EDGES = [32, 33, 47, 48, 49, 63, 64, 65, 97, 128, 129]
 
 
 @pytest.mark.parametrize("slots,last", [(40, 0), (33, 37), (33, 38)], ids=["streaming", "at_the_line", "past_it"])
-@pytest.mark.parametrize("H,I", [(256, 128), (512, 640), (1024, 384)])
+@pytest.mark.parametrize("H,I", [(256, 128), (512, 640), (1024, 384), (256, 5376)])
 def test_streaming_tile_edges(rng, H, I, slots, last):
     from mimo_stream import MoEBlock, Router, pools
     counts = EDGES + [0] * (slots - len(EDGES) - 1) + [last]
