@@ -14,7 +14,8 @@
  *
  * Workspaces: entry points that take (ws, ws_bytes) need a caller-owned device buffer of at least the size
  * the matching *_workspace_size() returns; its contents need no initialisation (every kernel writes what it
- * later reads).  Calls that share one workspace must be ordered on one stream.
+ * later reads).  The need never falls as M or T grows (other arguments equal), so one buffer of the largest size
+ * serves every smaller call.  Calls that share one workspace must be ordered on one stream.
  *
  * Device status: the fused entry points (mimo_moe_decode, mimo_moe_prefill, mimo_moe_prefill_block,
  * mimo_moe_layer_decode, mimo_moe_layer_prefill) take an optional status_out, a device int32 [1] that the
@@ -217,7 +218,7 @@ size_t mimo_moe_layer_prefill_workspace_size(int T, int E, int k, int n_slots, i
  * workspace in a scratch array the library holds on each GPU (MIMO_NOALLOC_SCRATCH_BYTES, kept until the process
  * ends); the call itself allocates nothing (per-kernel event timing is skipped for it).  Batches whose workspace
  * (mimo_moe_layer_decode_workspace_size) exceeds the scratch are refused with MIMO_ERR_WORKSPACE; MiMo's largest,
- * 8 rows of 256 experts, needs about 2.3 MB.  Every call on one GPU uses that GPU's one scratch array: calls that
+ * 8 rows of 256 experts, needs about 2.2 MB.  Every call on one GPU uses that GPU's one scratch array: calls that
  * overlap on one GPU (two host threads, or two streams without an ordering between them) race. */
 #define MIMO_NOALLOC_SCRATCH_BYTES (4u << 20)
 int mimo_moe_layer_decode_noalloc(const uint16_t* x, int M, const uint16_t* norm_w, float eps, const uint16_t* Wg,

@@ -9,11 +9,11 @@
 // the registers of the one wave that uses them and are turned into bf16 there (exactly: an E2M1 value times a power
 // of two); the bf16 activation rows, which all four waves use, go through an LDS ring.
 //
-// What bounds it: up to ~700 tokens HBM (512 tokens: gate/up and down read 3.4 GB in ~690 us, 5 TB/s; the loads alone
-// take 405 of gate/up's 460 us); above, the MFMAs at the ~1.9 GHz that the chip's power leaves (60% busy at 6250
+// What bounds it: up to ~700 tokens HBM (512 tokens: gate/up and down read 3.4 GB in ~680 us, 5 TB/s; the loads alone
+// took 405 us of gate/up's 460, now 438); above, the MFMAs at the ~1.9 GHz that the chip's power leaves (60% busy at 6250
 // tokens) and the copies that they hide only in part (gate/up 1516 us; without activation copies 1327, without weight
-// loads 1296, without both 1184).  A layer step took 369 / 779 / 1246 / 2807 us at 24 / 512 / 2048 / 6250 tokens with
-// two E4M3 planes per activation on the block-scaled MFMA and two launches per GEMM, and takes 301 / 716 / 1081 / 2392.
+// loads 1296, without both 1184).  A layer step took 379 / 775 / 1273 / 2839 us at 24 / 512 / 2048 / 6250 tokens with
+// two E4M3 planes per activation on the block-scaled MFMA and two launches per GEMM, and takes 313 / 702 / 1102 / 2431.
 #include <algorithm>
 #include <atomic>
 
@@ -48,7 +48,9 @@ struct PrefillArgs {
 // of the routes, so the pairing is right whatever order the unit sums in.
 //
 // In LDS the 16-byte chunk 4 g + m of route r sits at position (4 m + g) ^ (r & 15) of its 256-byte row: the operand
-// reads are then free of bank conflicts (with the chunk 4 g + m at (4 g + m) ^ (r & 15) they took twice the cycles).
+// reads are then free of bank conflicts (with the chunk 4 g + m at (4 g + m) ^ (r & 15) they took twice the cycles).  The
+// scale bytes are not: 16 rows of 32 bytes, 8 cycles a read, 6 of them conflicts, for 4 reads a step (0.18 to 0.39 conflict
+// cycles per access cycle over the kernels).
 constexpr int PF_NARROW_MAX = 32;
 constexpr int PF_WIDE_ROWS = 128;
 // Routes per slot up to which the streaming configuration runs (three blocks per CU, tiles of up to 64 routes), against

@@ -47,7 +47,8 @@ int launch_router_select(const float* logits, const float* bias, int T, int E, i
                          hipStream_t st, bool parts = false);
 // Logits of a chunk of at most kRlPartsMax tokens as kRlParts partial sums [kRlParts, T, E], which
 // launch_router_select(parts) adds; router_logits_parts: whether the inputs allow it.
-// Beyond, the blocks of whole reductions fill the chip: 512 tokens 16.4 us in parts, 27 whole; 1024 tokens 30 and 27.
+// Beyond, the blocks of whole reductions fill the chip: 512 tokens 14.8 us in parts, 25.5 whole; 640 20.0 and 25.3, 768
+// 20.7 and 25.6, 1024 26.8 and 25.6, and the selection takes 0.5 to 1.4 us more to add the parts.
 constexpr int kRlPartsMax = 640, kRlParts = 8;
 bool router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H);
 int launch_router_logits_parts(const uint16_t* x, const uint16_t* W, int T, int H, int E, float* part, hipStream_t st,

@@ -726,8 +726,8 @@ __global__ void __launch_bounds__(512) router_logits_mfma_kernel(const uint16_t*
 
 // The same products for chunks of few tokens, where blocks of 64 experts and the whole reduction are too few: a block
 // (4 waves) takes 32 tokens x 64 experts and one K-range of the 8, a wave 16 of the experts, and the partial sums go to
-// part [8, T, E].  A block's loads bound both kernels: with 24 tokens 4 blocks of 768 KB each took 24.6 us, 32 blocks of
-// 96 KB take 8.7; with 512, 29 and 17.9.  Each partial is summed as router_logits_mfma_kernel sums it and the selection
+// part [8, T, E].  A block's loads bound both kernels: with 24 tokens 4 blocks of 768 KB each take 25.4 us, 32 blocks of
+// 96 KB 8.4; with 512, 25.5 and 14.8.  Each partial is summed as router_logits_mfma_kernel sums it and the selection
 // adds them in the same order, so the logits are the same bits.
 __global__ void __launch_bounds__(256) router_logits_parts_kernel(const uint16_t* __restrict__ x,
                                                                   const uint16_t* __restrict__ W, int T, int H, int E,
